@@ -12,9 +12,12 @@
 //          vector loads, cross-lane combine with shuffles.
 //   split  long rows and few outputs: blocks reduce row chunks into partials
 //          in scratch, a second kernel combines them.
-//   thread one thread per output walking n in index order (strided rows,
-//          scans, float products, *_n_ind): adjacent threads read adjacent
-//          addresses when the broadcast dim 0 is the contiguous one.
+//   grid   strided rows and rows shorter than a wave: a block's threads cover
+//          outputs x positions along n, n cut into chunks where the outputs
+//          alone leave the chip idle (partials combined as for split).
+//   thread one thread per output walking n in index order (scans, float
+//          products, *_n_ind): adjacent threads read adjacent addresses when
+//          the broadcast dim 0 is the contiguous one.
 //
 // Semantics kept exactly: integer sums/products wrap in the output type
 // (any order gives PDL's bits), min/max follow PDL's rules (a NaN never
@@ -138,19 +141,117 @@ __global__ __launch_bounds__(RT) void red_split1(const Tin *__restrict__ a, RedP
   }
 }
 
-// stage 2: one wave per row combines its chunk partials
+// the R partials of each output, `step` apart in sh, meet in a tree; the
+// result is in the thread with r == 0
+template <int OP, class Tin, class Tacc>
+__device__ inline void block_tree(Part<Tin, Tacc> &pt, Part<Tin, Tacc> *sh, bool in, int r, int R, int step) {
+  sh[threadIdx.x] = pt;
+  for (int h = R > 1 ? 1 << (31 - __builtin_clz(R - 1)) : 0; h >= 1; h >>= 1) {
+    __syncthreads();
+    if (in && r < h && r + h < R) {
+      part_combine<OP>(pt, sh[threadIdx.x + h * step]);
+      sh[threadIdx.x] = pt;
+    }
+  }
+}
+
+// stage 2: G threads (a power of two, about four chunks each) combine the
+// partials of one row.  A wave per row walked 2048 chunks 32 to a lane, one
+// dependent load after another, and made half of a column sum (41 us, now 25).
 template <int OP, class Tin, class Tout, class Tacc, bool BAD>
-__global__ __launch_bounds__(RT) void red_split2(RedPlan p, int64_t nchunk, const Part<Tin, Tacc> *parts, Outs o) {
-  const int lane = threadIdx.x & 63;
-  const int64_t e = (int64_t)blockIdx.x * (RT / 64) + (threadIdx.x >> 6);
-  if (e >= p.nout) return;
-  int64_t off[MAXP];
-  out_offsets(p, e, off);
+__global__ __launch_bounds__(RT) void red_split2(RedPlan p, int64_t nchunk, int G, const Part<Tin, Tacc> *parts,
+                                                 Outs o) {
+  __shared__ Part<Tin, Tacc> sh[RT];
+  const int r = threadIdx.x % G;
+  const int64_t e = (int64_t)blockIdx.x * (RT / G) + threadIdx.x / G;
+  const bool in = e < p.nout;
   Part<Tin, Tacc> pt;
   part_init<OP, Tin, Tacc>(pt);
-  for (int64_t k = lane; k < nchunk; k += 64) part_combine<OP>(pt, parts[e * nchunk + k]);
-  wave_reduce<OP, Tin, Tacc>(pt);
-  if (lane == 0) part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
+  if (in) {
+#pragma unroll 4
+    for (int64_t k = r; k < nchunk; k += G) part_combine<OP>(pt, parts[e * nchunk + k]);
+  }
+  block_tree<OP>(pt, sh, in, r, G, 1);
+  if (in && r == 0) {
+    int64_t off[MAXP];
+    out_offsets(p, e, off);
+    part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
+  }
+}
+
+template <int OP, class Tin, class Tout, class Tacc, bool BAD>
+static void split2_launch(const RedPlan &p, int64_t nchunk, const Part<Tin, Tacc> *parts, const Outs &o,
+                          hipStream_t s) {
+  int G = 1;
+  while (G < RT && G * 4 < nchunk) G *= 2;
+  const int64_t per = RT / G;
+  hipLaunchKernelGGL((red_split2<OP, Tin, Tout, Tacc, BAD>), dim3((unsigned)((p.nout + per - 1) / per)), dim3(RT), 0, s,
+                     p, nchunk, G, parts, o);
+}
+
+// ---------------------------------------------------------------- grid
+// A block covers LE outputs x R positions along n (LE * R <= 256 threads):
+// thread (e, r) takes elements r, r + R, ... of its chunk of row e, eight
+// loads in flight, then the R partials of an output meet in a tree in LDS.
+// NFAST puts n on neighbouring threads (rows whose stride along n is the
+// smaller one, such as short unit-stride rows and stepped slices), otherwise
+// outputs are neighbours (columns of a table), so that a wave reads
+// neighbouring addresses either way.  Bound by HBM; one thread per output
+// walking n took 187 ms (0.5 GB/s) to average 24 columns of 1000003 floats,
+// this takes 25 us with the combine (19.3 + 5.4, 4.9 TB/s in this kernel).
+constexpr int GRID_U = 8;
+template <int OP, class Tin, class Tout, class Tacc, bool BAD, bool NFAST>
+__global__ __launch_bounds__(RT) void red_grid(const Tin *__restrict__ a, RedPlan p, Outs o, BadInfo ba, int LE, int R,
+                                               int64_t nchunk, int64_t clen, Part<Tin, Tacc> *parts) {
+  __shared__ Part<Tin, Tacc> sh[RT];
+  const Tin abv = bv_as<Tin>(ba.bv);
+  const int r = NFAST ? threadIdx.x % R : threadIdx.x / LE, el = NFAST ? threadIdx.x / R : threadIdx.x % LE;
+  const int64_t k = blockIdx.x % nchunk;
+  const int64_t cb = k * clen, ce = (cb + clen < p.n) ? cb + clen : p.n;
+  const int64_t ngroup = (p.nout + LE - 1) / LE;
+  for (int64_t gr = blockIdx.x / nchunk; gr < ngroup; gr += gridDim.x / nchunk) {
+    const int64_t e = gr * LE + el;
+    const bool in = e < p.nout && r < R && el < LE;
+    int64_t off[MAXP];
+    Part<Tin, Tacc> pt;
+    part_init<OP, Tin, Tacc>(pt);
+    if (in) {
+      out_offsets(p, e, off);
+      const Tin *ap = a + off[0];
+      const int64_t inc = p.inc_n[0];
+      int64_t i = cb + r;
+      for (; i + (int64_t)(GRID_U - 1) * R < ce; i += (int64_t)GRID_U * R) {
+        Tin x[GRID_U];
+#pragma unroll
+        for (int u = 0; u < GRID_U; u++) x[u] = ap[(i + (int64_t)u * R) * inc];
+#pragma unroll
+        for (int u = 0; u < GRID_U; u++) {
+          if constexpr (BAD) { if (isbad(x[u], abv, ba.isnan)) continue; }
+          part_push<OP, Tin, Tacc>(pt, x[u], i + (int64_t)u * R);
+        }
+      }
+      // the rest, fewer than GRID_U of them: loaded together as well
+      Tin x[GRID_U];
+#pragma unroll
+      for (int u = 0; u < GRID_U - 1; u++) {
+        const int64_t q = i + (int64_t)u * R;
+        x[u] = q < ce ? ap[q * inc] : Tin(0);
+      }
+#pragma unroll
+      for (int u = 0; u < GRID_U - 1; u++) {
+        const int64_t q = i + (int64_t)u * R;
+        if (q >= ce) continue;
+        if constexpr (BAD) { if (isbad(x[u], abv, ba.isnan)) continue; }
+        part_push<OP, Tin, Tacc>(pt, x[u], q);
+      }
+    }
+    block_tree<OP>(pt, sh, in, r, R, NFAST ? 1 : LE);
+    if (in && r == 0) {
+      if (nchunk == 1) part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
+      else parts[e * nchunk + k] = pt;
+    }
+    __syncthreads();   // sh is refilled for the next group
+  }
 }
 
 // ---------------------------------------------------------------- scan
@@ -309,20 +410,66 @@ __global__ __launch_bounds__(RT) void red_thread(const Tin *__restrict__ a, RedP
       Tout v = (Tout)tmp;
       if (BAD && !any) v = bv_as<Tout>(o.bv[0]);
       put<Tout>(o.p[0], off[1], v);
-    } else {
-      Part<Tin, Tacc> pt;
-      part_init<OP, Tin, Tacc>(pt);
-      for (int64_t i = 0; i < n; i++) {
-        Tin x = ap[i * ia];
-        if constexpr (BAD) { if (isbad(x, abv, ba.isnan)) continue; }
-        part_push<OP, Tin, Tacc>(pt, x, i);
-      }
-      part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
     }
   }
 }
 
 // ---------------------------------------------------------------- dispatch
+// launches red_grid: lanes along n where its stride is the smaller of the
+// two, a wave's worth of outputs side by side otherwise; n is cut into chunks
+// of at least 32 elements per thread until there are about 1024 blocks (four
+// per CU; 2048 measured 22.5 + 7.0 us for that table).  Without scratch for
+// the partials (a capture with none cached, the allocation-free entry's
+// limit) n stays whole and every call still runs.
+template <int OP, class Tin, class Tout, class Tacc, bool BAD>
+static hipError_t grid_launch(const RedPlan &p, const Tin *a, const Outs &o, const BadInfo &ba, hipStream_t s) {
+  const int64_t in0 = p.inc_n[0] < 0 ? -p.inc_n[0] : p.inc_n[0];
+  const int64_t ie0 = p.nd == 0 || p.nout == 1 ? INT64_MAX : (p.inc[0][0] < 0 ? -p.inc[0][0] : p.inc[0][0]);
+  const bool nfast = in0 < ie0;
+  int LE, R;
+  if (nfast) {
+    // at least four elements per thread before a second thread helps
+    R = 1;
+    while (R < 64 && R * 4 < p.n) R *= 2;
+    LE = RT / R;
+    if (p.nout < LE) {   // fewer outputs than that: more threads along n
+      LE = (int)p.nout;
+      while (R * 2 * LE <= RT && R * 4 < p.n) R *= 2;
+    }
+  } else {
+    LE = p.nout < 64 ? (int)p.nout : 64;
+    R = RT / LE;
+  }
+  const int64_t ngroup = (p.nout + LE - 1) / LE;
+  int64_t nchunk = (1024 + ngroup - 1) / ngroup;
+  const int64_t most = p.n / ((int64_t)R * 32);
+  nchunk = nchunk < most ? nchunk : most;
+  if (p.scratch) {
+    const int64_t fit = p.scratch_bytes / (int64_t)(sizeof(Part<Tin, Tacc>) * (size_t)p.nout);
+    nchunk = nchunk < fit ? nchunk : fit;
+  }
+  Part<Tin, Tacc> *parts = nullptr;
+  if (nchunk > 1) {
+    parts = (Part<Tin, Tacc> *)(p.scratch ? p.scratch : scratch_alloc(sizeof(*parts) * (size_t)p.nout * (size_t)nchunk));
+    if (!parts) nchunk = 1;
+  } else {
+    nchunk = 1;
+  }
+  int64_t clen = (p.n + nchunk - 1) / nchunk;
+  clen = clen < 1 ? 1 : clen;
+  const int64_t blocks = (ngroup < (1 << 20) ? ngroup : (1 << 20)) * nchunk;
+  if (nfast)
+    hipLaunchKernelGGL((red_grid<OP, Tin, Tout, Tacc, BAD, true>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
+                       LE, R, nchunk, clen, parts);
+  else
+    hipLaunchKernelGGL((red_grid<OP, Tin, Tout, Tacc, BAD, false>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o,
+                       ba, LE, R, nchunk, clen, parts);
+  if (parts) split2_launch<OP, Tin, Tout, Tacc, BAD>(p, nchunk, parts, o, s);
+  const hipError_t err = hipGetLastError();
+  if (parts && !p.scratch) scratch_free(parts);
+  return err;
+}
+
 template <int OP, class Tin, class Tout, class Tacc, bool BAD>
 static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, const BadInfo &ba, int *flag,
                              hipStream_t s) {
@@ -358,8 +505,7 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
         else
           hipLaunchKernelGGL((red_split1<OP, Tin, Tout, Tacc, BAD, 1>), dim3((unsigned)(p.nout * nchunk)), dim3(RT),
                              0, s, a, p, nchunk, clen, parts, ba, stream);
-        hipLaunchKernelGGL((red_split2<OP, Tin, Tout, Tacc, BAD>), dim3((unsigned)((p.nout + 3) / 4)), dim3(RT), 0, s,
-                           p, nchunk, parts, o);
+        split2_launch<OP, Tin, Tout, Tacc, BAD>(p, nchunk, parts, o, s);
         hipError_t err = hipGetLastError();
         if (!p.scratch) scratch_free(parts);
         return err;
@@ -374,19 +520,21 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
                            ba, stream);
       return hipGetLastError();
     }
-  }
-  if constexpr ((OP == R_CUMUSUM || OP == R_CUMUPROD) && !IsFloat<Tout>::v) {
-    if (p.inc_n[0] == 1 && p.inc_n[1] == 1 && p.n >= 256) {
-      int64_t blocks = p.nout < 65536 ? p.nout : 65536;
-      hipLaunchKernelGGL((scan_rows<OP, Tin, Tout, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba);
-      return hipGetLastError();
+    return grid_launch<OP, Tin, Tout, Tacc, BAD>(p, a, o, ba, s);
+  } else {
+    if constexpr ((OP == R_CUMUSUM || OP == R_CUMUPROD) && !IsFloat<Tout>::v) {
+      if (p.inc_n[0] == 1 && p.inc_n[1] == 1 && p.n >= 256) {
+        int64_t blocks = p.nout < 65536 ? p.nout : 65536;
+        hipLaunchKernelGGL((scan_rows<OP, Tin, Tout, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba);
+        return hipGetLastError();
+      }
     }
+    int64_t blocks = (p.nout + RT - 1) / RT;
+    if (blocks > 65536) blocks = 65536;
+    hipLaunchKernelGGL((red_thread<OP, Tin, Tout, Tacc, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
+                       flag);
+    return hipGetLastError();
   }
-  int64_t blocks = (p.nout + RT - 1) / RT;
-  if (blocks > 65536) blocks = 65536;
-  hipLaunchKernelGGL((red_thread<OP, Tin, Tout, Tacc, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
-                     flag);
-  return hipGetLastError();
 }
 
 template <int OP, class Tin, class Tout, class Tacc>
