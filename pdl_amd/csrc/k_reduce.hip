@@ -8,9 +8,9 @@
 //   minmaximum                  Ufunc.pd:563-613
 //
 // Kernels:
-//   wave   one 64-lane wavefront per output (rows with unit stride), 16-byte
+//   wave   1, 4 or 16 wavefronts per output (rows with unit stride), 16-byte
 //          vector loads, cross-lane combine with shuffles.
-//   split  long rows and few outputs: blocks reduce row chunks into partials
+//   split  the longest rows and few outputs: blocks reduce row chunks into partials
 //          in scratch, a second kernel combines them.
 //   grid   strided rows and rows shorter than a wave: a block's threads cover
 //          outputs x positions along n, n cut into chunks where the outputs
@@ -47,98 +47,104 @@ __device__ inline void out_offsets(const RedPlan &p, int64_t e, int64_t *off) {
   }
 }
 
-// ---------------------------------------------------------------- wave
+// ---------------------------------------------------------------- rows
 constexpr int RT = 256;  // threads per block (4 waves)
 
-template <int OP, class Tin, class Tout, class Tacc, bool BAD, int VEC>
-__device__ inline void row_segment(Part<Tin, Tacc> &pt, const Tin *__restrict__ a, int64_t o, int64_t begin,
-                                   int64_t end, int64_t inc, int lane, const BadInfo &ba, bool stream) {
-  const Tin abv = bv_as<Tin>(ba.bv);
-  int64_t i = begin + (int64_t)lane * VEC;
+// lane of NL cooperating lanes takes its share of elements [begin, end) of a
+// unit-stride row: the elements up to the first 16-byte boundary one to a
+// lane, then 16-byte vectors, then the rest one to a lane, each lane's in
+// increasing index order.  (Rows of odd length start unaligned; loading those
+// an element at a time took 167 us for 64 rows of 32091 ints.)
+template <int OP, class Tin, class Tacc, bool BAD, int NL>
+__device__ inline void row_segment(Part<Tin, Tacc> &pt, const Tin *__restrict__ row, int64_t begin, int64_t end,
+                                   int lane, const BadInfo &ba, bool stream) {
+  constexpr int VEC = 16 / sizeof(Tin);
   // 16-byte loads in flight per lane: 4 for 4- and 8-byte elements, 2 for
   // the narrower ones (eight or sixteen elements per load already)
   constexpr int RED_U = sizeof(Tin) >= 4 ? 4 : 2;
-  if constexpr (VEC > 1) {
-    // begin is a multiple of VEC and the row start is 16-byte aligned; RED_U
-    // vectors in flight per lane, consumed in increasing index order
-    for (; i + (RED_U - 1) * 64 * VEC + VEC <= end; i += RED_U * 64 * VEC) {
-      Vec<Tin, VEC> x[RED_U];
+  const Tin abv = bv_as<Tin>(ba.bv);
+  const int64_t lead = ((16 - (int)((uintptr_t)(row + begin) & 15)) & 15) / sizeof(Tin);
+  const int64_t vb = begin + lead < end ? begin + lead : end, ve = vb + (end - vb) / VEC * VEC;
+  auto push = [&](Tin x, int64_t i) {
+    if constexpr (BAD) { if (isbad(x, abv, ba.isnan)) return; }
+    part_push<OP, Tin, Tacc>(pt, x, i);
+  };
+  if (begin + lane < vb) push(row[begin + lane], begin + lane);
+  int64_t i = vb + (int64_t)lane * VEC;
+  for (; i + (RED_U - 1) * NL * VEC < ve; i += RED_U * NL * VEC) {
+    Vec<Tin, VEC> x[RED_U];
 #pragma unroll
-      for (int u = 0; u < RED_U; u++)
-        x[u] = stream ? load_nt<Tin, VEC>(a + o + i + u * 64 * VEC)
-                      : *reinterpret_cast<const Vec<Tin, VEC> *>(a + o + i + u * 64 * VEC);
+    for (int u = 0; u < RED_U; u++)
+      x[u] = stream ? load_nt<Tin, VEC>(row + i + u * NL * VEC)
+                    : *reinterpret_cast<const Vec<Tin, VEC> *>(row + i + u * NL * VEC);
 #pragma unroll
-      for (int u = 0; u < RED_U; u++)
+    for (int u = 0; u < RED_U; u++)
 #pragma unroll
-        for (int k = 0; k < VEC; k++) {
-          if constexpr (BAD) { if (isbad(x[u].v[k], abv, ba.isnan)) continue; }
-          part_push<OP, Tin, Tacc>(pt, x[u].v[k], i + u * 64 * VEC + k);
-        }
-    }
-    for (; i + VEC <= end; i += 64 * VEC) {
-      Vec<Tin, VEC> x = stream ? load_nt<Tin, VEC>(a + o + i) : *reinterpret_cast<const Vec<Tin, VEC> *>(a + o + i);
+      for (int k = 0; k < VEC; k++) push(x[u].v[k], i + u * NL * VEC + k);
+  }
+  for (; i < ve; i += NL * VEC) {
+    const Vec<Tin, VEC> x = stream ? load_nt<Tin, VEC>(row + i) : *reinterpret_cast<const Vec<Tin, VEC> *>(row + i);
 #pragma unroll
-      for (int k = 0; k < VEC; k++) {
-        if constexpr (BAD) { if (isbad(x.v[k], abv, ba.isnan)) continue; }
-        part_push<OP, Tin, Tacc>(pt, x.v[k], i + k);
-      }
-    }
-    // tail: fewer than VEC*64 elements remain past the vector loop's reach
-    for (int64_t t = ((end - begin) / VEC) * VEC + begin + lane; t < end; t += 64) {
-      Tin x = a[o + t];
-      if constexpr (BAD) { if (isbad(x, abv, ba.isnan)) continue; }
-      part_push<OP, Tin, Tacc>(pt, x, t);
-    }
-  } else {
-    for (; i < end; i += 64) {
-      Tin x = a[o + i * inc];
-      if constexpr (BAD) { if (isbad(x, abv, ba.isnan)) continue; }
-      part_push<OP, Tin, Tacc>(pt, x, i);
-    }
+    for (int k = 0; k < VEC; k++) push(x.v[k], i + k);
+  }
+  if (ve + lane < end) push(row[ve + lane], ve + lane);
+}
+
+// the NW waves of a block join their partials (each already combined within
+// the wave); the result is in thread 0
+template <int OP, class Tin, class Tacc, int NW>
+__device__ inline void waves_join(Part<Tin, Tacc> &pt, Part<Tin, Tacc> *sh) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (lane == 0) sh[w] = pt;
+  __syncthreads();
+  if (w == 0) {
+    part_init<OP, Tin, Tacc>(pt);
+    if (lane < NW) pt = sh[lane];
+    wave_reduce<OP, Tin, Tacc>(pt);
   }
 }
 
-template <int OP, class Tin, class Tout, class Tacc, bool BAD, int VEC>
-__global__ __launch_bounds__(RT) void red_wave(const Tin *__restrict__ a, RedPlan p, Outs o, BadInfo ba,
-                                               bool stream) {
-  const int lane = threadIdx.x & 63;
-  const int64_t nw = (int64_t)gridDim.x * (RT / 64);
-  for (int64_t e = (int64_t)blockIdx.x * (RT / 64) + (threadIdx.x >> 6); e < p.nout; e += nw) {
+// NW waves per row; four rows per block of 256 threads for NW = 1, else a
+// row per block
+template <int OP, class Tin, class Tout, class Tacc, bool BAD, int NW>
+__global__ __launch_bounds__(NW > 4 ? NW * 64 : RT) void red_wave(const Tin *__restrict__ a, RedPlan p, Outs o,
+                                                                  BadInfo ba, bool stream) {
+  constexpr int PER = NW == 1 ? 4 : 1;
+  __shared__ Part<Tin, Tacc> sh[NW];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int64_t e = (int64_t)blockIdx.x * PER + (NW == 1 ? w : 0); e < p.nout; e += (int64_t)gridDim.x * PER) {
     int64_t off[MAXP];
     out_offsets(p, e, off);
     Part<Tin, Tacc> pt;
     part_init<OP, Tin, Tacc>(pt);
-    row_segment<OP, Tin, Tout, Tacc, BAD, VEC>(pt, a, off[0], 0, p.n, p.inc_n[0], lane, ba, stream);
+    row_segment<OP, Tin, Tacc, BAD, NW * 64>(pt, a + off[0], 0, p.n, NW == 1 ? lane : (int)threadIdx.x, ba, stream);
     wave_reduce<OP, Tin, Tacc>(pt);
-    if (lane == 0) part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
+    if constexpr (NW > 1) {
+      waves_join<OP, Tin, Tacc, NW>(pt, sh);
+      if (threadIdx.x == 0) part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
+      __syncthreads();   // sh is refilled for the next row
+    } else {
+      if (lane == 0) part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
+    }
   }
 }
 
 // ---------------------------------------------------------------- split
 // stage 1: block (e, k) reduces chunk k of row e into parts[e * nchunk + k]
-template <int OP, class Tin, class Tout, class Tacc, bool BAD, int VEC>
+template <int OP, class Tin, class Tout, class Tacc, bool BAD>
 __global__ __launch_bounds__(RT) void red_split1(const Tin *__restrict__ a, RedPlan p, int64_t nchunk, int64_t clen,
                                                  Part<Tin, Tacc> *parts, BadInfo ba, bool stream) {
   __shared__ Part<Tin, Tacc> sh[RT / 64];
   const int64_t e = blockIdx.x / nchunk, k = blockIdx.x % nchunk;
   int64_t off[MAXP];
   out_offsets(p, e, off);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int64_t cb = k * clen, ce = (cb + clen < p.n) ? cb + clen : p.n;
   Part<Tin, Tacc> pt;
   part_init<OP, Tin, Tacc>(pt);
-  // the 4 waves of the block take interleaved sub-chunks of the chunk
-  const int64_t sub = ((ce - cb) + 3) / 4;
-  const int64_t subr = ((sub + VEC - 1) / VEC) * VEC;
-  const int64_t sb = cb + w * subr, se = (sb + subr < ce) ? sb + subr : ce;
-  if (sb < se) row_segment<OP, Tin, Tout, Tacc, BAD, VEC>(pt, a, off[0], sb, se, p.inc_n[0], lane, ba, stream);
+  row_segment<OP, Tin, Tacc, BAD, RT>(pt, a + off[0], cb, ce, threadIdx.x, ba, stream);
   wave_reduce<OP, Tin, Tacc>(pt);
-  if (lane == 0) sh[w] = pt;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int j = 1; j < RT / 64; j++) part_combine<OP>(pt, sh[j]);
-    parts[blockIdx.x] = pt;
-  }
+  waves_join<OP, Tin, Tacc, RT / 64>(pt, sh);
+  if (threadIdx.x == 0) parts[blockIdx.x] = pt;
 }
 
 // the R partials of each output, `step` apart in sh, meet in a tree; the
@@ -478,16 +484,15 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
   constexpr bool SEQ = SCAN || OP == R_MIN_N_IND || OP == R_MAX_N_IND || (is_prod(OP) && IsFloat<Tacc>::v);
   if constexpr (!SEQ) {
     if (p.n >= 64 && p.inc_n[0] == 1) {
-      constexpr int VEC = 16 / sizeof(Tin);
-      bool aligned = ((uintptr_t)(a + p.off[0]) % 16 == 0);
-      for (int d = 0; d < p.nd; d++) aligned = aligned && (p.inc[0][d] % VEC == 0);
       const bool stream = streaming_read((size_t)p.n * (size_t)p.nout * sizeof(Tin));
-      if (p.nout < 1024 && p.n >= 65536) {
-        // long rows, few outputs: split each row into chunks
+      const size_t row_bytes = (size_t)p.n * sizeof(Tin);
+      if (p.nout < 512 && row_bytes >= ((size_t)512 << 10)) {
+        // long rows, few outputs: about 2048 chunks in all, of 32 KiB or more
         int64_t want = (2048 + p.nout - 1) / p.nout;
         int64_t clen = (p.n + want - 1) / want;
-        if (clen < 16384) clen = 16384;
-        clen = ((clen + VEC * 256 - 1) / (VEC * 256)) * (VEC * 256);
+        const int64_t least = (32 << 10) / (int64_t)sizeof(Tin);
+        if (clen < least) clen = least;
+        clen = (clen + RT - 1) / RT * RT;   // a multiple of the 16-byte vectors' length
         int64_t nchunk = (p.n + clen - 1) / clen;
         // partials in the caller's scratch when it brings one, else from the cache
         const size_t need = sizeof(Part<Tin, Tacc>) * (size_t)p.nout * (size_t)nchunk;
@@ -499,25 +504,29 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
           parts = (Part<Tin, Tacc> *)scratch_alloc(need);
           if (!parts) return hipErrorOutOfMemory;
         }
-        if (aligned)
-          hipLaunchKernelGGL((red_split1<OP, Tin, Tout, Tacc, BAD, VEC>), dim3((unsigned)(p.nout * nchunk)), dim3(RT),
-                             0, s, a, p, nchunk, clen, parts, ba, stream);
-        else
-          hipLaunchKernelGGL((red_split1<OP, Tin, Tout, Tacc, BAD, 1>), dim3((unsigned)(p.nout * nchunk)), dim3(RT),
-                             0, s, a, p, nchunk, clen, parts, ba, stream);
+        hipLaunchKernelGGL((red_split1<OP, Tin, Tout, Tacc, BAD>), dim3((unsigned)(p.nout * nchunk)), dim3(RT), 0, s, a,
+                           p, nchunk, clen, parts, ba, stream);
         split2_launch<OP, Tin, Tout, Tacc, BAD>(p, nchunk, parts, o, s);
         hipError_t err = hipGetLastError();
         if (!p.scratch) scratch_free(parts);
         return err;
       }
-      int64_t blocks = (p.nout + 3) / 4;
-      if (blocks > 65536) blocks = 65536;
-      if (aligned)
-        hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, VEC>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o,
-                           ba, stream);
-      else
-        hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 1>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o,
-                           ba, stream);
+      // a wave per row where the rows fill the chip (sixteen waves per CU) or
+      // are short; else enough waves per row, each with about four 16-byte
+      // loads per lane
+      const int64_t loads = (int64_t)(row_bytes / 16 / 64);
+      if (p.nout >= 4096 || loads < 8) {
+        int64_t blocks = (p.nout + 3) / 4;
+        if (blocks > 65536) blocks = 65536;
+        hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 1>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
+                           stream);
+      } else if (p.nout >= 1024 || loads < 32) {
+        hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 4>), dim3((unsigned)p.nout), dim3(RT), 0, s, a, p, o, ba,
+                           stream);
+      } else {
+        hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 16>), dim3((unsigned)p.nout), dim3(16 * 64), 0, s, a, p,
+                           o, ba, stream);
+      }
       return hipGetLastError();
     }
     return grid_launch<OP, Tin, Tout, Tacc, BAD>(p, a, o, ba, s);
