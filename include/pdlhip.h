@@ -351,7 +351,7 @@ pdlhip_error pdlhip_graph_destroy(void *graph);
  *   SPLIT16   default; float: FP16 hi/lo split, 3 MFMA products, FP32
  *             accumulate (single products from 64 per side; broadcast batches
  *             of products with 16..64 per side; other shapes as FP32);
- *             double: FP64 MFMA for single products of about 1024^2 and up
+ *             double: FP64 MFMA from 8 per side
  *   FP32      plain SIMT kernel with fused multiply-add (float and double)
  *   PDLORDER  SIMT, multiply then add in ascending t: bit-identical to the
  *             reference's loop
@@ -383,8 +383,8 @@ pdlhip_error pdlhip_readdata(const char *op, int datatype, int bvalflag,
 
 /* Autotuner (no reference counterpart; PDL picks its CPU split with a
  * static rule, pdlbroadcast.c:95-159).  Kernel variants (list tiles, float
- * GEMM block shapes, the engine of mid-size double products) are timed
- * once per shape class and kept in $PDLHIP_TUNE_FILE (default
+ * GEMM block shapes) are timed once per shape class and kept in
+ * $PDLHIP_TUNE_FILE (default
  * ~/.cache/pdlhip/tune-<arch>.txt); PDLHIP_TUNE=0 keeps the default rules.
  * The counts of choices this process measured and reused from the file. */
 pdlhip_error pdlhip_tune_stats(int64_t *measured, int64_t *reused);

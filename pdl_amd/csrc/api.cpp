@@ -1124,18 +1124,14 @@ static pdlhip_error readdata(const Sig &s, int T, bool bad, const Brc &b, pdlhip
     }
     if (g.defer) g.defer->missed++;
     // the autotuner's block shape for float products on the matrix cores
-    // (128x128 or 256x256) and engine for mid-size double products (SIMT 1
-    // or FP64 matrix cores 2), timed into a scratch output
+    // (128x128 or 256x256), timed into a scratch output
     const bool mm16 = T == PDLHIP_F && (g.mm_mode == PDLHIP_MM_SPLIT16 || g.mm_mode == PDLHIP_MM_FP8);
-    const int64_t nb128 = ((p.H + 127) / 128) * ((p.W + 127) / 128);
-    const bool f64mid = T == PDLHIP_D && g.mm_mode != PDLHIP_MM_PDLORDER && g.mm_mode != PDLHIP_MM_FP32 &&
-                        p.nbatch == 1 && p.H >= 64 && p.W >= 64 && p.T >= 16 && nb128 >= 16 && nb128 < 256;
-    if (!bad && p.nbatch == 1 && ((mm16 && p.H >= 512 && p.W >= 512 && p.T >= 32) || f64mid)) {
+    if (!bad && p.nbatch == 1 && mm16 && p.H >= 512 && p.W >= 512 && p.T >= 32) {
       char fam[160];
       snprintf(fam, sizeof fam, "matmult:%s:%s:h2^%d:w2^%d:t2^%d", type_name(T),
                g.mm_mode == PDLHIP_MM_FP8 ? "fp8" : "default", ilog2(p.H), ilog2(p.W), ilog2(p.T));
-      std::vector<int> cands = mm16 ? std::vector<int>{128, 256} : std::vector<int>{1, 2};
-      const int dflt = mm16 ? ((p.H >= 1024 && p.W >= 1024) ? 256 : 128) : (nb128 >= 64 ? 2 : 1);
+      const std::vector<int> cands = {128, 256};
+      const int dflt = (p.H >= 1024 && p.W >= 1024) ? 256 : 128;
       void *tc = nullptr;
       auto run_one = [&](int cand) -> hipError_t {
         if (!tc) tc = dev_alloc((size_t)p.H * p.W * type_size(T));
