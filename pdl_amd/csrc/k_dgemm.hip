@@ -7,14 +7,15 @@
 // small: 64x64 of C per block of 4 waves keeps four blocks resident per CU,
 // whose waves cover each other's loads and barriers, and cuts a product into
 // enough blocks for 256 CUs.  4096^3: 2.09 ms, 65.8 TFLOP/s (128x128 blocks of
-// the same kernel 2.33 ms, 128x64 2.28); 1500^3: 148 us (before, 144 blocks of
-// 128x128: 280 us; 123 where the operands change from call to call); 512^3: 18 us (the SIMT kernel: 85).  Operands go global ->
-// registers -> LDS in stages of 16 k, two stages' loads in flight while the
-// matrix cores work on a third (one: 59 instead of 54 us at 1024^3, where a
-// CU has one block).  LDS holds rows of 16 k, padded
-// to 18 doubles: a lane reads two neighbouring k of its row as 16 bytes (eight
-// rows fall on distinct bank groups) and feeds them to two instructions; which
-// k an instruction covers is free as long as A and B agree.
+// the same kernel 2.33 ms, 128x64 2.28); 1500^3: 148 us (123 where the operands
+// change from call to call; before, 144 blocks of 128x128: 280); 512^3: 18 us
+// (the SIMT kernel: 85).  Operands go global -> registers -> LDS in stages of
+// 16 k, two stages' loads in flight while the matrix cores work on a third
+// (one: 59 instead of 54 us at 1024^3, where a CU has one block).  LDS holds
+// rows of 16 k, padded to 18 doubles: a lane reads two neighbouring k of its
+// row as 16 bytes (eight rows fall on distinct bank groups) and feeds them to
+// two instructions; which k an instruction covers is free as long as A and B
+// agree.
 //
 // Tiles that would fill only part of the chip in the last wave of blocks are
 // cut along t into S parts, each summed into scratch, and joined by a second

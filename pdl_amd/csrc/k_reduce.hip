@@ -15,9 +15,11 @@
 //   grid   strided rows and rows shorter than a wave: a block's threads cover
 //          outputs x positions along n, n cut into chunks where the outputs
 //          alone leave the chip idle (partials combined as for split).
-//   thread one thread per output walking n in index order (scans, float
-//          products, *_n_ind): adjacent threads read adjacent addresses when
-//          the broadcast dim 0 is the contiguous one.
+//   scan   integer scans of unit-stride rows: blocks scan chunks through LDS.
+//   seq    scans in PDL's order: a lane per row in LDS, other waves moving.
+//   thread one thread per output walking n in index order (float products,
+//          *_n_ind): adjacent threads read adjacent addresses when the
+//          broadcast dim 0 is the contiguous one.
 //
 // Semantics kept exactly: integer sums/products wrap in the output type
 // (any order gives PDL's bits), min/max follow PDL's rules (a NaN never
@@ -266,12 +268,33 @@ __global__ __launch_bounds__(RT) void red_grid(const Tin *__restrict__ a, RedPla
 // of 16 elements per thread, then wave and block prefix combines.  Wrapping
 // integer + and * are associative, so the result has PDL's exact bits.  A bad
 // element contributes the identity and is written as the output's bad value
-// (Ufunc.pd:127-132).
+// (Ufunc.pd:127-132).  Few long rows are cut into chunks of a multiple of 4096
+// elements, a block each: scan_totals leaves every chunk's total, and a
+// chunk's scan starts from the totals before it (16 rows of 1000000 ints:
+// 520 us with a block per row, 13 + 24 with chunks).
 constexpr int SC_IT = 16, SC_CH = RT * SC_IT;
 __device__ inline int sc_pad(int i) { return i + (i >> 4); }
 
 template <int OP, class Tin, class Tout, bool BAD>
-__global__ __launch_bounds__(RT) void scan_rows(const Tin *__restrict__ a, RedPlan p, Outs o, BadInfo ba) {
+__global__ __launch_bounds__(RT) void scan_totals(const Tin *__restrict__ a, RedPlan p, BadInfo ba, int64_t nchunk,
+                                                  int64_t clen, Tout *totals) {
+  constexpr int ROP = OP == R_CUMUPROD ? R_PROD : R_SUM;
+  __shared__ Part<Tin, Tout> sh[RT / 64];
+  const int64_t e = blockIdx.x / nchunk, k = blockIdx.x % nchunk;
+  int64_t off[MAXP];
+  out_offsets(p, e, off);
+  const int64_t cb = k * clen, ce = cb + clen < p.n ? cb + clen : p.n;
+  Part<Tin, Tout> pt;
+  part_init<ROP, Tin, Tout>(pt);
+  row_segment<ROP, Tin, Tout, BAD, RT>(pt, a + off[0], cb, ce, threadIdx.x, ba, false);
+  wave_reduce<ROP, Tin, Tout>(pt);
+  waves_join<ROP, Tin, Tout, RT / 64>(pt, sh);
+  if (threadIdx.x == 0) totals[blockIdx.x] = pt.s;
+}
+
+template <int OP, class Tin, class Tout, bool BAD>
+__global__ __launch_bounds__(RT) void scan_rows(const Tin *__restrict__ a, RedPlan p, Outs o, BadInfo ba, int64_t nchunk,
+                                                int64_t clen, const Tout *totals) {
   constexpr bool PR = (OP == R_CUMUPROD);
   __shared__ Tout sh[SC_CH + SC_CH / 16];
   __shared__ uint8_t badm[BAD ? SC_CH : 1];
@@ -280,14 +303,30 @@ __global__ __launch_bounds__(RT) void scan_rows(const Tin *__restrict__ a, RedPl
   const Tin abv = bv_as<Tin>(ba.bv);
   const Tout obv = bv_as<Tout>(o.bv[0]);
   const Tout ident = PR ? Tout(1) : Tout(0);
-  for (int64_t e = blockIdx.x; e < p.nout; e += gridDim.x) {
+  for (int64_t q = blockIdx.x; q < p.nout * nchunk; q += gridDim.x) {
+    const int64_t e = nchunk == 1 ? q : q / nchunk, k = q - e * nchunk;
     int64_t off[MAXP];
     out_offsets(p, e, off);
     const Tin *ap = a + off[0];
     Tout *bp = (Tout *)o.p[0] + off[1];
     Tout carry = ident;
-    for (int64_t c0 = 0; c0 < p.n; c0 += SC_CH) {
-      const int len = (p.n - c0 < SC_CH) ? (int)(p.n - c0) : SC_CH;
+    if (k > 0) {   // the totals of the row's chunks before this one
+      Tout t = ident;
+      for (int64_t i = tid; i < k; i += RT) t = PR ? wmul(t, totals[e * nchunk + i]) : wadd(t, totals[e * nchunk + i]);
+#pragma unroll
+      for (int m = 32; m >= 1; m >>= 1) {
+        const Tout u = shfl_xor(t, m);
+        t = PR ? wmul(t, u) : wadd(t, u);
+      }
+      if (lane == 0) wsum[w] = t;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < RT / 64; i++) carry = PR ? wmul(carry, wsum[i]) : wadd(carry, wsum[i]);
+      __syncthreads();
+    }
+    const int64_t end = (k + 1) * clen < p.n ? (k + 1) * clen : p.n;
+    for (int64_t c0 = k * clen; c0 < end; c0 += SC_CH) {
+      const int len = (end - c0 < SC_CH) ? (int)(end - c0) : SC_CH;
       // every load of the chunk is issued before the first LDS write
       Tin xv[SC_IT];
 #pragma unroll
@@ -354,6 +393,230 @@ __global__ __launch_bounds__(RT) void scan_rows(const Tin *__restrict__ a, RedPl
   }
 }
 
+// Scans in PDL's own order, element after element (float and double sums and
+// products, whose rounding that order defines; Ufunc.pd:120-140), and scans
+// of short or strided rows of any type.  The chain of one row is serial, so
+// this is bound by it until there are rows enough to be bound by HBM.  In a
+// block three waves bring in the next chunk of C elements of each of G rows
+// and store the one before (along whichever of n and rows is the closer in
+// memory) while the first wave scans:
+//   G > 1   a lane per row, out of LDS and back, 16 bytes at a time
+//   one row the lanes hold the chunk in registers, K neighbours each, and add
+//           in turn, so that the chain has no LDS access in it (9 cycles
+//           per element against 15.4 through LDS)
+// One thread per row straight from memory took 52.4 ms for a row of 476006
+// floats, this takes 1.8 ms; 60000 rows of 256: 27 us (4.6 TB/s).
+constexpr int SQ_MOVERS = RT - 64;
+template <class Tout> constexpr int SQ_E = 8192 / (int)sizeof(Tout);   // elements of a chunk, at most
+template <class Tout> constexpr int SQ_K = SQ_E<Tout> / 64;            // one row: neighbours per lane
+// a row of a chunk in LDS: 16 bytes after each row (or each lane's K
+// elements) spread what the lanes read at once over the banks
+template <class T, class Tout> constexpr int sq_pitch(int C, bool one) {
+  return C + 16 / (int)sizeof(T) * (one ? C / SQ_K<Tout> : 1);
+}
+
+// lane l's v, in every lane
+template <class T> __device__ inline T lane_value(T v, int l) {
+  static_assert(sizeof(T) == 4 || sizeof(T) == 8, "one or two registers");
+  int w[sizeof(T) / 4];
+  __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+  for (int i = 0; i < (int)sizeof(T) / 4; i++) w[i] = __builtin_amdgcn_readlane(w[i], l);
+  __builtin_memcpy(&v, w, sizeof(T));
+  return v;
+}
+
+template <int OP, class Tin, class Tout, bool BAD, bool ONE>
+__global__ __launch_bounds__(RT) void scan_seq(const Tin *__restrict__ a, RedPlan p, Outs o, BadInfo ba, int G, int C,
+                                               int in_nfast, int out_nfast) {
+  constexpr bool PR = (OP == R_CUMUPROD || OP == R_DCUMUPROD);
+  constexpr int IT = 16, VI = 16 / (int)sizeof(Tin), VO = 16 / (int)sizeof(Tout);
+  extern __shared__ __align__(16) char sq_lds[];
+  const int pi = sq_pitch<Tin, Tout>(C, ONE), po = sq_pitch<Tout, Tout>(C, ONE);
+  constexpr int K = SQ_K<Tout>;
+  // [row offsets in a and in b][2 chunks of Tout][2 chunks of Tin]; pointers are
+  // formed from sq_lds where they are used, which keeps them LDS pointers
+  // (through a table of buffers they turn generic, and the scan three times slower)
+  int64_t *rowa = (int64_t *)sq_lds, *rowb = rowa + G;
+  auto out = [&](int64_t k) { return (Tout *)(sq_lds + 16 * G) + (int)(k & 1) * G * po; };
+  auto in = [&](int64_t k) { return (Tin *)(sq_lds + 16 * G + 2 * G * po * sizeof(Tout)) + (int)(k & 1) * G * pi; };
+  const int tid = threadIdx.x, lc = __builtin_ctz(C), lg = __builtin_ctz(G);
+  const int64_t e0 = (int64_t)blockIdx.x * G;
+  const int rows = p.nout - e0 < G ? (int)(p.nout - e0) : G;
+  if (tid < rows) {
+    int64_t off[MAXP];
+    out_offsets(p, e0 + tid, off);
+    rowa[tid] = off[0];
+    rowb[tid] = off[1];
+  }
+  __syncthreads();
+  const int64_t ia = p.inc_n[0], ib = p.inc_n[1], nc = (p.n + C - 1) / C;
+  const Tin abv = bv_as<Tin>(ba.bv);
+  const Tout obv = bv_as<Tout>(o.bv[0]);
+  // position idx of a chunk -> row and element
+  auto where = [&](int idx, int nfast, int &r, int &c) {
+    r = nfast ? idx >> lc : idx & (G - 1);
+    c = nfast ? idx & (C - 1) : idx >> lg;
+  };
+  // a mover's share of a chunk, all of its loads in flight at once (past the
+  // rows' end the last element again: scanned after it, never stored)
+  constexpr int U = SQ_E<Tout> / SQ_MOVERS + 1;
+  const int me = tid - 64;
+  Tin x[U];
+  auto load = [&](int64_t k) {
+    const int64_t c0 = k * C;
+    const int clast = p.n - c0 < C ? (int)(p.n - c0) - 1 : C - 1;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = me + u * SQ_MOVERS;
+      int r, c;
+      where(i < G * C ? i : G * C - 1, in_nfast, r, c);
+      x[u] = a[rowa[r < rows ? r : rows - 1] + (c0 + (c < clast ? c : clast)) * ia];
+    }
+  };
+  auto commit = [&](int64_t k) {
+    Tin *dst = in(k);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = me + u * SQ_MOVERS;
+      int r, c;
+      where(i, in_nfast, r, c);
+      if (i < G * C) dst[ONE ? c + c / K * VI : r * pi + c] = x[u];
+    }
+  };
+  auto store = [&](int64_t k) {
+    const int64_t c0 = k * C;
+    const int len = p.n - c0 < C ? (int)(p.n - c0) : C;
+    const Tout *src = out(k);
+    const auto bp = as_global((Tout *)o.p[0]);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i = me + u * SQ_MOVERS;
+      int r, c;
+      where(i, out_nfast, r, c);
+      if (i < G * C && r < rows && c < len) bp[rowb[r] + (c0 + c) * ib] = src[ONE ? c + c / K * VO : r * po + c];
+    }
+  };
+  if (tid >= 64) {
+    load(0);
+    commit(0);
+    if (nc > 1) load(1);
+  }
+  __syncthreads();
+  Tout run = PR ? Tout(1) : Tout(0);
+  for (int64_t k = 0; k <= nc; k++) {
+    if (tid >= 64) {
+      if (k + 1 < nc) commit(k + 1);
+      if (k + 2 < nc) load(k + 2);
+      if (k > 0) store(k - 1);
+    } else if (ONE) {
+      if (k < nc) {
+        // what lies past the row's end is scanned last and not stored
+        const int len = p.n - k * C < C ? (int)(p.n - k * C) : C;
+        const Tin *src = in(k) + tid * (K + VI);
+        Tout *dst = out(k) + tid * (K + VO);
+        Tout v[K];
+        unsigned skip = 0;
+        if (tid * K < C) {
+#pragma unroll
+          for (int q = 0; q < K; q += VI) {
+            const Vec<Tin, VI> t = *reinterpret_cast<const Vec<Tin, VI> *>(src + q);
+#pragma unroll
+            for (int i = 0; i < VI; i++) {
+              v[q + i] = (Tout)t.v[i];
+              if constexpr (BAD) skip |= isbad(t.v[i], abv, ba.isnan) ? 1u << (q + i) : 0u;
+            }
+          }
+        }
+        for (int l = 0; l * K < len; l++) {
+          if (tid == l) {
+#pragma unroll
+            for (int i = 0; i < K; i++) {
+              const Tout next = PR ? wmul(run, v[i]) : wadd(run, v[i]);
+              const bool sk = BAD && (skip >> i & 1);
+              run = sk ? run : next;
+              v[i] = sk ? obv : run;
+            }
+          }
+          run = lane_value(run, l);
+        }
+        if (tid * K < C) {
+#pragma unroll
+          for (int q = 0; q < K; q += VO) {
+            Vec<Tout, VO> t;
+#pragma unroll
+            for (int i = 0; i < VO; i++) t.v[i] = v[q + i];
+            *reinterpret_cast<Vec<Tout, VO> *>(dst + q) = t;
+          }
+        }
+      }
+    } else if (tid < rows && k < nc) {
+      // whole groups of 16: what lies past the row's end is scanned last and not stored
+      const Tin *src = in(k) + tid * pi;
+      Tout *dst = out(k) + tid * po;
+      const int len = p.n - k * C < C ? (int)(p.n - k * C) : C;
+      Vec<Tin, VI> x[IT / VI];
+#pragma unroll
+      for (int v = 0; v < IT / VI; v++) x[v] = *reinterpret_cast<const Vec<Tin, VI> *>(src + v * VI);
+      for (int c = 0; c < len; c += IT) {
+        // 16 bytes of the wider type at a time: scan, store, and fetch the
+        // elements of the next group that come to the same place.  In this
+        // order an LDS access issues while the chain waits for its last sum.
+        const int cn = c + IT < len ? c + IT : c;
+        constexpr int VG = VI > VO ? VI : VO;
+#pragma unroll
+        for (int q = 0; q < IT; q += VG) {
+          Vec<Tout, VO> y[VG / VO];
+#pragma unroll
+          for (int i = 0; i < VG; i++) {
+            const Tin xi = x[(q + i) / VI].v[(q + i) % VI];
+            bool skip = false;
+            if constexpr (BAD) skip = isbad(xi, abv, ba.isnan);
+            const Tout next = PR ? wmul(run, (Tout)xi) : wadd(run, (Tout)xi);
+            run = skip ? run : next;
+            y[i / VO].v[i % VO] = skip ? obv : run;
+          }
+#pragma unroll
+          for (int v = 0; v < VG / VO; v++) *reinterpret_cast<Vec<Tout, VO> *>(dst + c + q + v * VO) = y[v];
+#pragma unroll
+          for (int v = 0; v < VG / VI; v++)
+            x[q / VI + v] = *reinterpret_cast<const Vec<Tin, VI> *>(src + cn + q + v * VI);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+template <int OP, class Tin, class Tout, bool BAD>
+static hipError_t seq_launch(const RedPlan &p, const Tin *a, const Outs &o, const BadInfo &ba, hipStream_t s) {
+  // rows per block: two blocks per CU before a block takes a second row; 8 KiB
+  // of outputs per chunk (37 KiB of LDS, four blocks per CU), no more than a
+  // row has
+  int G = 1;
+  while (G < 64 && (int64_t)G * 2 * 512 <= p.nout) G *= 2;
+  constexpr int E = SQ_E<Tout>;
+  int C = E / G;
+  while (C > 32 && C / 2 >= p.n) C /= 2;
+  // more rows where they are short
+  while (G < 64 && G * C * 2 <= E && (int64_t)G * 2 * 256 <= p.nout) G *= 2;
+  const bool one = G == 1;
+  auto mag = [](int64_t x) { return x < 0 ? -x : x; };
+  auto nfast = [&](int q) { return p.nout == 1 || p.nd == 0 || mag(p.inc_n[q]) <= mag(p.inc[q][0]); };
+  const size_t lds = 16 * (size_t)G + 2 * (size_t)G * (sizeof(Tin) * sq_pitch<Tin, Tout>(C, one) +
+                                                       sizeof(Tout) * sq_pitch<Tout, Tout>(C, one));
+  const int64_t blocks = (p.nout + G - 1) / G;
+  if (blocks >= ((int64_t)1 << 31)) return hipErrorInvalidConfiguration;
+  if (one)
+    hipLaunchKernelGGL((scan_seq<OP, Tin, Tout, BAD, true>), dim3((unsigned)blocks), dim3(RT), lds, s, a, p, o, ba, G, C,
+                       nfast(0) ? 1 : 0, nfast(1) ? 1 : 0);
+  else
+    hipLaunchKernelGGL((scan_seq<OP, Tin, Tout, BAD, false>), dim3((unsigned)blocks), dim3(RT), lds, s, a, p, o, ba, G, C,
+                       nfast(0) ? 1 : 0, nfast(1) ? 1 : 0);
+  return hipGetLastError();
+}
+
 // ---------------------------------------------------------------- thread
 template <int OP, class Tin, class Tout, class Tacc, bool BAD>
 __global__ __launch_bounds__(RT) void red_thread(const Tin *__restrict__ a, RedPlan p, Outs o, BadInfo ba,
@@ -364,20 +627,7 @@ __global__ __launch_bounds__(RT) void red_thread(const Tin *__restrict__ a, RedP
     out_offsets(p, e, off);
     const Tin *ap = a + off[0];
     const int64_t n = p.n, ia = p.inc_n[0];
-    if constexpr (OP == R_CUMUSUM || OP == R_DCUMUSUM || OP == R_CUMUPROD || OP == R_DCUMUPROD) {
-      // Ufunc.pd:120-140 in index order (PDL's exact rounding for floats)
-      Tout *bp = (Tout *)o.p[0] + off[1];
-      const int64_t ib = p.inc_n[1];
-      const Tout obv = bv_as<Tout>(o.bv[0]);
-      constexpr bool PR = (OP == R_CUMUPROD || OP == R_DCUMUPROD);
-      Tout tmp = PR ? Tout(1) : Tout(0);
-      for (int64_t i = 0; i < n; i++) {
-        Tin x = ap[i * ia];
-        if constexpr (BAD) { if (isbad(x, abv, ba.isnan)) { bp[i * ib] = obv; continue; } }
-        tmp = PR ? wmul(tmp, (Tout)x) : wadd(tmp, (Tout)x);
-        bp[i * ib] = tmp;
-      }
-    } else if constexpr (OP == R_MIN_N_IND || OP == R_MAX_N_IND) {
+    if constexpr (OP == R_MIN_N_IND || OP == R_MAX_N_IND) {
       // Ufunc.pd:484-540: m passes, each skipping indices already chosen
       int64_t *cp = (int64_t *)o.p[0] + off[1];
       const int64_t ic = p.inc_m, m = p.m;
@@ -530,14 +780,35 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
       return hipGetLastError();
     }
     return grid_launch<OP, Tin, Tout, Tacc, BAD>(p, a, o, ba, s);
-  } else {
+  } else if constexpr (SCAN) {
     if constexpr ((OP == R_CUMUSUM || OP == R_CUMUPROD) && !IsFloat<Tout>::v) {
       if (p.inc_n[0] == 1 && p.inc_n[1] == 1 && p.n >= 256) {
-        int64_t blocks = p.nout < 65536 ? p.nout : 65536;
-        hipLaunchKernelGGL((scan_rows<OP, Tin, Tout, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba);
-        return hipGetLastError();
+        // rows of several chunks are cut while they alone leave CUs idle:
+        // about 2048 blocks in all, each of at least 8192 elements
+        int64_t nchunk = 1, clen = p.n;
+        Tout *totals = nullptr;
+        if (p.nout < 512 && p.n >= 32768) {
+          int64_t want = (2048 + p.nout - 1) / p.nout;
+          clen = (p.n + want - 1) / want;
+          clen = clen < 8192 ? 8192 : (clen + SC_CH - 1) / SC_CH * SC_CH;
+          nchunk = (p.n + clen - 1) / clen;
+          totals = (Tout *)scratch_alloc(sizeof(Tout) * (size_t)(p.nout * nchunk));
+          if (!totals) { nchunk = 1; clen = p.n; }   // none cached during a capture: a block per row
+        }
+        if (totals)
+          hipLaunchKernelGGL((scan_totals<OP, Tin, Tout, BAD>), dim3((unsigned)(p.nout * nchunk)), dim3(RT), 0, s, a, p,
+                             ba, nchunk, clen, totals);
+        const int64_t blocks = p.nout * nchunk < 65536 ? p.nout * nchunk : 65536;
+        hipLaunchKernelGGL((scan_rows<OP, Tin, Tout, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba, nchunk,
+                           clen, totals);
+        const hipError_t err = hipGetLastError();
+        if (totals) scratch_free(totals);
+        return err;
       }
     }
+    if (p.n == 0) return hipSuccess;
+    return seq_launch<OP, Tin, Tout, BAD>(p, a, o, ba, s);
+  } else {
     int64_t blocks = (p.nout + RT - 1) / RT;
     if (blocks > 65536) blocks = 65536;
     hipLaunchKernelGGL((red_thread<OP, Tin, Tout, Tacc, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
