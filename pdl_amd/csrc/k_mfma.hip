@@ -36,14 +36,13 @@
 
 #include "device.hpp"
 #include "launch.hpp"
+#include "mfma_common.hpp"
 
 namespace pdlhip {
 
 void *scratch_alloc(size_t bytes);
 void scratch_free(void *p);
 
-typedef _Float16 half_t;
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int MB = 128, NB = 128, KB = 32, KPAD = KB + 8;
@@ -54,9 +53,6 @@ __device__ __forceinline__ float fin_abs(float x) {
   return a < __builtin_inff() ? a : 0.0f;
 }
 
-// exponent of a power of two held as a normal float
-__device__ __forceinline__ int pow2_exp(float s) { return ((__float_as_int(s) >> 23) & 0xff) - 127; }
-
 // hi/lo split of a scaled element y (finite), and the part of its
 // representation error beyond 2^-22 |y| (both differences are exact)
 __device__ __forceinline__ float split_hilo(float y, half_t &h, half_t &l) {
@@ -65,24 +61,6 @@ __device__ __forceinline__ float split_hilo(float y, half_t &h, half_t &l) {
   l = (half_t)r1;
   const float e = fabsf(r1 - (float)l) - 0x1p-22f * fabsf(y);
   return e > 0.0f ? e : 0.0f;
-}
-
-// Whether output c (unscaled; the accumulator was c * 2^e) must come from
-// PDL's loop: the range-loss bound (D_A[h] + D_B[w]) * 2^15 (scaled units)
-// exceeds 2^-22 |c|, or c is not finite.  The GEMM epilogue and the fixup
-// kernel evaluate the same test on the same stored c.
-__device__ __forceinline__ bool mm_needs_fix(float c, float dd, int e) {
-  if (dd == 0.0f && fabsf(c) < __builtin_inff()) return false;
-  return !(ldexpf(dd * 32768.0f, -e) <= 0x1p-22f * fabsf(c));
-}
-
-// the GEMM epilogue for one output: unscale the accumulator exactly and
-// mark the row of an output the fixup kernel must recompute
-__device__ __forceinline__ float mm_finish(float v, float da, float db, float sa, float sb, int *rowflag, int64_t h) {
-  const int e = pow2_exp(sa) + pow2_exp(sb);
-  const float c = ldexpf(v, -e);
-  if (mm_needs_fix(c, da + db, e)) rowflag[h] = 1;   // the same value from every writer
-  return c;
 }
 
 // power of two that brings max|row| into [2^(e-1), 2^e) with e = target
@@ -190,10 +168,11 @@ __global__ __launch_bounds__(256) void make_scales(float *s, float *d, int *rowf
 }
 
 // packs 8 consecutive k of one row: hi/lo FP16 (or e4m3) of x * sc with
-// non-finite elements as zero; returns their range-loss excess (scaled
-// units; +Inf if any element is non-finite, which FP8 tracks alone)
+// non-finite elements as zero, to their place in the panels; returns their
+// range-loss excess (scaled units; +Inf if any element is non-finite, which
+// FP8 tracks alone)
 template <bool FP8>
-__device__ __forceinline__ float pack8(const float (&x)[8], float sc, half_t *hi, half_t *lo, uint8_t *q8) {
+__device__ __forceinline__ float pack8(const float (&x)[8], float sc, half_t *hl, uint8_t *q8) {
   float ex = 0.0f;
   float y[8];
 #pragma unroll
@@ -219,8 +198,8 @@ __device__ __forceinline__ float pack8(const float (&x)[8], float sc, half_t *hi
       vh[i] = h;
       vl[i] = l;
     }
-    *reinterpret_cast<half8 *>(hi) = vh;
-    *reinterpret_cast<half8 *>(lo) = vl;
+    *reinterpret_cast<half8 *>(hl) = vh;
+    *reinterpret_cast<half8 *>(hl + PIECE) = vl;
   }
   return ex;
 }
@@ -231,8 +210,7 @@ template <bool FP8>
 __global__ __launch_bounds__(256) void pack_tile(const float *__restrict__ src, int64_t o, int64_t inc_r,
                                                  int64_t inc_k, int64_t R, int64_t K, int64_t Kp,
                                                  const float *__restrict__ scale, float *__restrict__ dsum,
-                                                 half_t *__restrict__ hi, half_t *__restrict__ lo,
-                                                 uint8_t *__restrict__ q8, int64_t ntk) {
+                                                 half_t *__restrict__ hl, uint8_t *__restrict__ q8, int64_t ntk) {
   __shared__ float t[64][65];
   const int64_t r0 = (blockIdx.x / ntk) * 64, k0 = (blockIdx.x % ntk) * 64;
   load_tile64<false>(t, src, o, inc_r, inc_k, R, K, r0, k0);
@@ -247,22 +225,22 @@ __global__ __launch_bounds__(256) void pack_tile(const float *__restrict__ src, 
     float x[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) x[i] = t[rr][kg + i];
-    const float ex = pack8<FP8>(x, sc, hi + gr * Kp + gk, lo + gr * Kp + gk, q8 + gr * Kp + gk);
+    const float ex = pack8<FP8>(x, sc, hl + panel_at(gr, gk, Kp), q8 + gr * Kp + gk);
     if (ex != 0.0f && gr < R) atomicAdd(&dsum[gr], ex);
   }
 }
 
 // pack an operand whose k index is unit-stride (rows 16-byte aligned): a
 // thread converts 8 consecutive k of one row (two 16-byte loads) into one
-// 16-byte hi and one lo store (8 bytes for FP8); zeros past R and K
+// 16-byte hi and one lo store (8 bytes for FP8); zeros past R and K.  FP16:
+// a block takes 32 rows x kchunk k in steps of 64, so that what it stores to a
+// piece fills whole lines; FP8: neighbouring threads along k.
 template <bool FP8>
 __global__ __launch_bounds__(256) void pack_rows(const float *__restrict__ src, int64_t o, int64_t inc_r, int64_t R,
                                                  int64_t K, int64_t Rp, int64_t Kp, const float *__restrict__ scale,
-                                                 float *__restrict__ dsum, half_t *__restrict__ hi,
-                                                 half_t *__restrict__ lo, uint8_t *__restrict__ q8) {
-  const int64_t ng = Kp / 8, total = Rp * ng;
-  for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < total; g += (int64_t)gridDim.x * 256) {
-    const int64_t row = g / ng, k0 = (g % ng) * 8;
+                                                 float *__restrict__ dsum, half_t *__restrict__ hl,
+                                                 uint8_t *__restrict__ q8, int64_t kchunk) {
+  auto one = [&](int64_t row, int64_t k0, float sc) {
     float x[8];
     if (row < R && k0 + 8 <= K) {
       const float *p = src + o + row * inc_r + k0;
@@ -274,8 +252,22 @@ __global__ __launch_bounds__(256) void pack_rows(const float *__restrict__ src, 
 #pragma unroll
       for (int i = 0; i < 8; i++) x[i] = (row < R && k0 + i < K) ? src[o + row * inc_r + k0 + i] : 0.0f;
     }
-    const float ex = pack8<FP8>(x, scale[row], hi + row * Kp + k0, lo + row * Kp + k0, q8 + row * Kp + k0);
+    const float ex = pack8<FP8>(x, sc, hl + panel_at(row, k0, Kp), q8 + row * Kp + k0);
     if (ex != 0.0f && row < R) atomicAdd(&dsum[row], ex);
+  };
+  if constexpr (FP8) {
+    const int64_t ng = Kp / 8, total = Rp * ng;
+    for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < total; g += (int64_t)gridDim.x * 256) {
+      const int64_t row = g / ng;
+      one(row, (g % ng) * 8, scale[row]);
+    }
+  } else {
+    const int64_t nkc = (Kp + kchunk - 1) / kchunk;
+    const int64_t row = blockIdx.x / nkc * 32 + threadIdx.x / 8, kb = blockIdx.x % nkc * kchunk;
+    const int64_t ke = kb + kchunk < Kp ? kb + kchunk : Kp;
+    const float sc = scale[row];
+#pragma unroll 2
+    for (int64_t k = kb + threadIdx.x % 8 * 8; k < ke; k += 64) one(row, k, sc);
   }
 }
 
@@ -288,144 +280,7 @@ __device__ inline void mm_batch_offsets_m(const MmPlan &p, int64_t bidx, int64_t
   }
 }
 
-// block -> C tile.  The 8 XCDs take blocks round-robin (block b runs on XCD
-// b % 8), so each XCD is given one contiguous share of the tile order; within
-// a share, tiles go in groups of 8 tile-rows, column by column, so the blocks
-// resident on one XCD at a time reuse the same A row-panels and B
-// column-panels from that XCD's L2.
-__device__ inline void tile_of(int64_t b, int64_t ntm, int64_t ntn, int64_t &tm, int64_t &tn) {
-  const int64_t nb = ntm * ntn;
-  const int64_t t = (nb % 8 == 0) ? (b % 8) * (nb / 8) + b / 8 : b;
-  constexpr int64_t G = 8;
-  const int64_t g = t / (G * ntn), r = t % (G * ntn);
-  const int64_t rows = ntm - g * G < G ? ntm - g * G : G;
-  tm = g * G + r % rows;
-  tn = r / rows;
-}
-
-// The operands stream into LDS with direct global->LDS loads
-// (global_load_lds_dwordx4: lane i of a wave writes 16 bytes at the wave's
-// LDS address + 16*i), no registers in between, over two stages: while the
-// matrix cores work on stage k, stage k+1 is being filled.  A wave computes
-// 64x64 of C as 2x2 tiles of v_mfma_f32_32x32x16_f16 (twice the work of the
-// 16x16x32 form per issue slot); the block 128x128.
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-template <class T> __device__ __forceinline__ void dma16(const T *g, T *l) {
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)g,
-                                   (__attribute__((address_space(3))) void *)l, 16, 0, 0);
-}
-
-// BM x BN block tile, NW = WR x WC waves, each wave (BM/WR) x (BN/WC) of C as
-// TI x TJ tiles of 32x32.  128x128 (4 waves, 2x2 tiles each) for smaller
-// products; 256x256 (8 waves, 2x4 tiles each) halves the bytes staged per
-// MFMA and gives each step enough work to cover the loads of the next.
-template <int BM, int BN, int WR, int WC>
-__global__ __launch_bounds__(WR * WC * 64) void split16_gemm(const half_t *__restrict__ Ahi,
-                                                             const half_t *__restrict__ Alo,
-                                                             const half_t *__restrict__ Bhi,
-                                                             const half_t *__restrict__ Blo,
-                                                             const float *__restrict__ sA,
-                                                             const float *__restrict__ sB,
-                                                             const float *__restrict__ dA,
-                                                             const float *__restrict__ dB, int *rowflag,
-                                                             float *__restrict__ c, MmPlan p, int64_t Kp,
-                                                             int64_t ntm, int64_t ntn) {
-  constexpr int NW = WR * WC, TI = BM / WR / 32, TJ = BN / WC / 32;
-  constexpr int RA = BM / NW, RB = BN / NW;   // rows of A / B each wave stages
-  static_assert(RA % 16 == 0 && RB % 16 == 0, "a wave stages whole 16-row loads");
-  // [stage][hi/lo][row][k]: rows of 32 halves (four 16-byte segments) with
-  // segment s of row r stored at s ^ ((r >> 1) & 3).  LDS serves 128 bytes
-  // (32 banks) per cycle, i.e. 8 lanes of a 16-byte access: the fragment
-  // reads (8 rows, one segment) then fall on distinct banks
-  __shared__ half_t lA[2][2][BM][KB];
-  __shared__ half_t lB[2][2][BN][KB];
-  auto sw = [](int row, int seg) { return ((seg ^ ((row >> 1) & 3)) * 8); };
-  int64_t tm, tn;
-  tile_of(blockIdx.x, ntm, ntn, tm, tn);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wr = w / WC, wc = w % WC;
-  const half_t *ah = Ahi + tm * BM * Kp, *al = Alo + tm * BM * Kp;
-  const half_t *bh = Bhi + tn * BN * Kp, *bl = Blo + tn * BN * Kp;
-  f32x16 acc[TI][TJ];
-#pragma unroll
-  for (int i = 0; i < TI; i++)
-#pragma unroll
-    for (int j = 0; j < TJ; j++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) acc[i][j][r] = 0.f;
-  // lane i of a 16-row load lands on row i/4, physical segment i%4, so it
-  // fetches that row's logical segment
-  const int drow = lane >> 2;
-  auto fill = [&](int st, int64_t k0) {
-#pragma unroll
-    for (int s = 0; s < RA / 16; s++) {
-      const int row = RA * w + 16 * s + drow;
-      const int64_t off = (int64_t)row * Kp + k0 + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
-      dma16(ah + off, &lA[st][0][RA * w + 16 * s][0]);
-      dma16(al + off, &lA[st][1][RA * w + 16 * s][0]);
-    }
-#pragma unroll
-    for (int s = 0; s < RB / 16; s++) {
-      const int row = RB * w + 16 * s + drow;
-      const int64_t off = (int64_t)row * Kp + k0 + ((lane & 3) ^ ((row >> 1) & 3)) * 8;
-      dma16(bh + off, &lB[st][0][RB * w + 16 * s][0]);
-      dma16(bl + off, &lB[st][1][RB * w + 16 * s][0]);
-    }
-  };
-  fill(0, 0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  int cur = 0;
-  // 32x32x16 operand layout: lane l holds row (l % 32), k (l / 32) * 8 .. +7
-  const int lr = lane & 31, lseg = lane >> 5;
-  for (int64_t k0 = 0; k0 < Kp; k0 += KB) {
-    // the other stage was last read in the previous step, before the barrier
-    if (k0 + KB < Kp) fill(cur ^ 1, k0 + KB);
-#pragma unroll
-    for (int ks = 0; ks < KB / 16; ks++) {
-      half8 fbh[TJ], fbl[TJ];
-#pragma unroll
-      for (int j = 0; j < TJ; j++) {
-        const int br = wc * 32 * TJ + j * 32 + lr;
-        fbh[j] = *reinterpret_cast<const half8 *>(&lB[cur][0][br][sw(br, ks * 2 + lseg)]);
-        fbl[j] = *reinterpret_cast<const half8 *>(&lB[cur][1][br][sw(br, ks * 2 + lseg)]);
-      }
-#pragma unroll
-      for (int i = 0; i < TI; i++) {
-        const int ar = wr * 32 * TI + i * 32 + lr;
-        const half8 fah = *reinterpret_cast<const half8 *>(&lA[cur][0][ar][sw(ar, ks * 2 + lseg)]);
-        const half8 fal = *reinterpret_cast<const half8 *>(&lA[cur][1][ar][sw(ar, ks * 2 + lseg)]);
-        // product by product over the row's TJ accumulators
-#pragma unroll
-        for (int j = 0; j < TJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fal, fbh[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < TJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fah, fbl[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-        for (int j = 0; j < TJ; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fah, fbh[j], acc[i][j], 0, 0, 0);
-      }
-    }
-    // the next stage's loads have landed and every wave is done with this one
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    cur ^= 1;
-  }
-  // D layout of a 32x32 tile: lane l, reg r -> row 8*(r/4) + 4*(l/32) + r%4, col l%32
-#pragma unroll
-  for (int i = 0; i < TI; i++)
-#pragma unroll
-    for (int j = 0; j < TJ; j++)
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int64_t h = tm * BM + wr * 32 * TI + i * 32 + 8 * (r / 4) + 4 * (lane >> 5) + (r & 3);
-        const int64_t wcol = tn * BN + wc * 32 * TJ + j * 32 + (lane & 31);
-        if (h < p.H && wcol < p.W)
-          c[p.off[2] + wcol * p.c_w + h * p.c_h] = mm_finish(acc[i][j][r], dA[h], dB[wcol], sA[h], sB[wcol],
-                                                             rowflag, h);
-      }
-}
-
-// FP8 e4m3: one product per tile, pipelined like split16_gemm
+// FP8 e4m3: one product per tile, one LDS stage filled from registers
 __global__ __launch_bounds__(256) void fp8_gemm(const uint8_t *__restrict__ A8, const uint8_t *__restrict__ B8,
                                                const float *__restrict__ sA, const float *__restrict__ sB,
                                                const float *__restrict__ dA, const float *__restrict__ dB,
@@ -483,9 +338,10 @@ __global__ __launch_bounds__(256) void fp8_gemm(const uint8_t *__restrict__ A8, 
 }
 
 // FP8 on v_mfma_scale_f32_32x32x64_f8f6f4 (e4m3 operands, unit block scales:
-// rows and columns are pre-scaled by powers of two as for split16), the same
-// DMA two-stage pipeline over 64-byte k-steps; 256x256 blocks of 8 waves,
-// each 64x128 of C as 2x4 tiles of 32x32.
+// rows and columns are pre-scaled by powers of two as for split16).  Operands
+// stream into LDS with direct global->LDS loads over two stages of 64-byte
+// k-steps: while the matrix cores work on one, the other is being filled;
+// 256x256 blocks of 8 waves, each 64x128 of C as 2x4 tiles of 32x32.
 typedef int i32x8 __attribute__((ext_vector_type(8)));
 constexpr int KB8 = 64;
 
@@ -683,8 +539,8 @@ __global__ __launch_bounds__(256) void mm_fixup(const float *a, const float *b, 
 }
 
 static hipError_t prep_operand(const float *src, int64_t o, int64_t inc_r, int64_t inc_k, int64_t R, int64_t K,
-                               int64_t Rp, int64_t Kp, float *scale, float *dsum, int *rowflag, half_t *hi,
-                               half_t *lo, uint8_t *q8, bool fp8, hipStream_t s) {
+                               int64_t Rp, int64_t Kp, float *scale, float *dsum, int *rowflag, half_t *hl,
+                               uint8_t *q8, bool fp8, hipStream_t s) {
   // rows along unit-stride k that start 16-byte aligned take the vector kernels
   const bool rows16 = inc_k == 1 && ((uintptr_t)(src + o) % 16 == 0) && inc_r % 4 == 0;
   if (rows16)
@@ -701,23 +557,28 @@ static hipError_t prep_operand(const float *src, int64_t o, int64_t inc_r, int64
   hipLaunchKernelGGL(make_scales, dim3((unsigned)((Rp + 255) / 256)), dim3(256), 0, s, scale, dsum, rowflag, R, Rp,
                      fp8 ? 8 : 15);
   if (rows16) {
-    int64_t blocks = (Rp * (Kp / 8) + 255) / 256;
-    blocks = blocks > 65536 ? 65536 : blocks;
-    if (fp8)
+    if (fp8) {
+      int64_t blocks = (Rp * (Kp / 8) + 255) / 256;
+      blocks = blocks > 65536 ? 65536 : blocks;
       hipLaunchKernelGGL((pack_rows<true>), dim3((unsigned)blocks), dim3(256), 0, s, src, o, inc_r, R, K, Rp, Kp, scale,
-                         dsum, hi, lo, q8);
-    else
-      hipLaunchKernelGGL((pack_rows<false>), dim3((unsigned)blocks), dim3(256), 0, s, src, o, inc_r, R, K, Rp, Kp,
-                         scale, dsum, hi, lo, q8);
+                         dsum, hl, q8, (int64_t)0);
+    } else {
+      // about 2048 blocks of 64 to 1024 k
+      int64_t kchunk = Rp / 32 * Kp / 2048;
+      kchunk = kchunk > 1024 ? 1024 : (kchunk + 63) / 64 * 64;
+      kchunk = kchunk < 64 ? 64 : kchunk;
+      hipLaunchKernelGGL((pack_rows<false>), dim3((unsigned)(Rp / 32 * ((Kp + kchunk - 1) / kchunk))), dim3(256), 0, s,
+                         src, o, inc_r, R, K, Rp, Kp, scale, dsum, hl, q8, kchunk);
+    }
     return hipGetLastError();
   }
   const int64_t ntr = (Rp + 63) / 64, ntk = (Kp + 63) / 64;
   if (fp8)
     hipLaunchKernelGGL((pack_tile<true>), dim3((unsigned)(ntr * ntk)), dim3(256), 0, s, src, o, inc_r, inc_k, R, K, Kp,
-                       scale, dsum, hi, lo, q8, ntk);
+                       scale, dsum, hl, q8, ntk);
   else
     hipLaunchKernelGGL((pack_tile<false>), dim3((unsigned)(ntr * ntk)), dim3(256), 0, s, src, o, inc_r, inc_k, R, K,
-                       Kp, scale, dsum, hi, lo, q8, ntk);
+                       Kp, scale, dsum, hl, q8, ntk);
   return hipGetLastError();
 }
 
@@ -970,21 +831,19 @@ hipError_t launch_mfma_f32(const MmPlan &p, const float *a, const float *b, floa
   float *sA = (float *)buf, *sB = sA + Hp, *dA = sB + Wp, *dB = dA + Hp;
   int *rowflag = (int *)(dB + Wp);
   char *q = buf + (head + 255) / 256 * 256;
-  half_t *Ahi = nullptr, *Alo = nullptr, *Bhi = nullptr, *Blo = nullptr;
+  half_t *Ah = nullptr, *Bh = nullptr;   // panels, hi and lo
   uint8_t *A8 = nullptr, *B8 = nullptr;
   if (fp8) {
     A8 = (uint8_t *)q;
     B8 = A8 + Hp * Kp;
   } else {
-    Ahi = (half_t *)q;
-    Alo = Ahi + Hp * Kp;
-    Bhi = Alo + Hp * Kp;
-    Blo = Bhi + Wp * Kp;
+    Ah = (half_t *)q;
+    Bh = Ah + 2 * Hp * Kp;
   }
   int64_t o[3] = {p.off[0], p.off[1], p.off[2]};
   // A rows = h (stride a_h), k = t (stride a_t); B "rows" = w (b_w), k = t (b_t)
-  hipError_t e = prep_operand(a, o[0], p.a_h, p.a_t, p.H, p.T, Hp, Kp, sA, dA, rowflag, Ahi, Alo, A8, fp8, s);
-  if (e == hipSuccess) e = prep_operand(b, o[1], p.b_w, p.b_t, p.W, p.T, Wp, Kp, sB, dB, nullptr, Bhi, Blo, B8, fp8, s);
+  hipError_t e = prep_operand(a, o[0], p.a_h, p.a_t, p.H, p.T, Hp, Kp, sA, dA, rowflag, Ah, A8, fp8, s);
+  if (e == hipSuccess) e = prep_operand(b, o[1], p.b_w, p.b_t, p.W, p.T, Wp, Kp, sB, dB, nullptr, Bh, B8, fp8, s);
   const int64_t ntm = Hp / BMr, ntn = Wp / BNr;
   if (e == hipSuccess) {
     if (fp8 && big)
@@ -993,12 +852,8 @@ hipError_t launch_mfma_f32(const MmPlan &p, const float *a, const float *b, floa
     else if (fp8)
       hipLaunchKernelGGL(fp8_gemm, dim3((unsigned)(ntm * ntn)), dim3(256), 0, s, A8, B8, sA, sB, dA, dB, rowflag, c,
                          p, Kp, ntm, ntn);
-    else if (big)
-      hipLaunchKernelGGL((split16_gemm<256, 256, 4, 2>), dim3((unsigned)(ntm * ntn)), dim3(512), 0, s, Ahi, Alo, Bhi,
-                         Blo, sA, sB, dA, dB, rowflag, c, p, Kp, ntm, ntn);
     else
-      hipLaunchKernelGGL((split16_gemm<128, 128, 2, 2>), dim3((unsigned)(ntm * ntn)), dim3(256), 0, s, Ahi, Alo, Bhi,
-                         Blo, sA, sB, dA, dB, rowflag, c, p, Kp, ntm, ntn);
+      launch_split16(big, Ah, Bh, sA, sB, dA, dB, rowflag, c, p, Kp, ntm, ntn, s);
     e = hipGetLastError();
   }
   if (e == hipSuccess) {
