@@ -43,7 +43,7 @@ def units():
     u.append(("k_mfma.hip", "mfma", []))
     # accumulators in VGPRs: the loop's matrix instructions otherwise copy
     # them to AGPRs and back every step
-    u.append(("k_dgemm.hip", "dgemm", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]))
+    u.append(("k_tile.hip", "tile", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]))
     u.append(("k_hgemm.hip", "hgemm", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]))
     u.append(("k_batch.hip", "batch", []))
     u.append(("k_ragged.hip", "ragged", []))

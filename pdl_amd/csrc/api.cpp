@@ -1123,15 +1123,19 @@ static pdlhip_error readdata(const Sig &s, int T, bool bad, const Brc &b, pdlhip
       return ok();
     }
     if (g.defer) g.defer->missed++;
-    // the autotuner's block shape for float products on the matrix cores
-    // (128x128 or 256x256), timed into a scratch output
+    // the autotuner's engine for float products: the FP32 matrix cores (64),
+    // or FP16 split / FP8 blocks of 128x128 or 256x256, timed into a scratch
+    // output
     const bool mm16 = T == PDLHIP_F && (g.mm_mode == PDLHIP_MM_SPLIT16 || g.mm_mode == PDLHIP_MM_FP8);
     if (!bad && p.nbatch == 1 && mm16 && p.H >= 512 && p.W >= 512 && p.T >= 32) {
       char fam[160];
       snprintf(fam, sizeof fam, "matmult:%s:%s:h2^%d:w2^%d:t2^%d", type_name(T),
-               g.mm_mode == PDLHIP_MM_FP8 ? "fp8" : "default", ilog2(p.H), ilog2(p.W), ilog2(p.T));
-      const std::vector<int> cands = {128, 256};
-      const int dflt = (p.H >= 1024 && p.W >= 1024) ? 256 : 128;
+               g.mm_mode == PDLHIP_MM_FP8 ? "fp8" : "tile_or_ring", ilog2(p.H), ilog2(p.W), ilog2(p.T));
+      std::vector<int> cands = {128, 256};
+      int dflt = (p.H >= 1024 && p.W >= 1024) ? 256 : 128;
+      const double flops = 2.0 * (double)p.H * (double)p.W * (double)p.T;
+      if (g.mm_mode == PDLHIP_MM_SPLIT16 && flops <= 3e10) cands.push_back(64);
+      if (g.mm_mode == PDLHIP_MM_SPLIT16 && flops <= 8e9) dflt = 64;
       void *tc = nullptr;
       auto run_one = [&](int cand) -> hipError_t {
         if (!tc) tc = dev_alloc((size_t)p.H * p.W * type_size(T));
