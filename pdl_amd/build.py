@@ -45,7 +45,7 @@ def units():
     # them to AGPRs and back every step
     u.append(("k_tile.hip", "tile", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]))
     u.append(("k_hgemm.hip", "hgemm", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]))
-    u.append(("k_batch.hip", "batch", []))
+    u.append(("k_batch.hip", "batch", ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]))
     u.append(("k_ragged.hip", "ragged", []))
     u.append(("api.cpp", "api", ["-x", "hip"]))
     return u

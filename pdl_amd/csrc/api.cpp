@@ -1439,7 +1439,7 @@ static pdlhip_error run(const Sig &s, pdlhip_pdl **user, int npdls, const int64_
 // Measured choices of kernel variants per shape class, kept in a text file
 // per GPU architecture so that later processes reuse them: one line per
 // entry, "<key> <choice>", the key naming the kernel family, element type,
-// shape class and architecture (e.g. "list:float:mfma1:dim2^8:items2^12:gfx950").
+// shape class and architecture (e.g. "list:float:tiles1:dim2^8:items2^12:gfx950").
 // The file is $PDLHIP_TUNE_FILE, else $XDG_CACHE_HOME/pdlhip/tune-<arch>.txt,
 // else $HOME/.cache/pdlhip/tune-<arch>.txt; PDLHIP_TUNE=0 turns timing off
 // (each family's default rule applies), PDLHIP_TUNE_VERBOSE=1 prints each
@@ -1545,7 +1545,8 @@ struct ListH {
   MmItem *d_items = nullptr;
   unsigned int *d_counter = nullptr;
   int3 *d_w32 = nullptr, *d_w64 = nullptr;
-  int tile = 64;        // 32 / 64: SIMT tiles; 0: the matrix-core kernel (64x64 work items)
+  unsigned long32 = 0, long64 = 0;   // work items of the longest bin
+  int tile = 64;        // 32 / 64: SIMT tiles; 0 / 2: the matrix cores, 64x64 / 32x32 work items; 1: BF16 split
   bool mfma = false;    // float/double list in a default mode whose items fit 32-bit offsets
 };
 
@@ -1558,10 +1559,11 @@ static void list_release(ListH &h) {
 }
 
 static hipError_t list_launch(const ListH &h, int tile, bool each) {
-  const std::vector<int3> &w = tile == 32 ? h.work32 : h.work64;   // the MFMA kernel takes 64x64 items
+  const bool small = tile == 32 || tile == 2;
+  const std::vector<int3> &w = small ? h.work32 : h.work64;
   const int nblocks = (int)std::max<size_t>(std::min<size_t>(w.size(), 2048), 1);
-  return launch_matmult_list(h.d.T, h.d_items, h.d.items.data(), (int)h.d.items.size(), tile == 32 ? h.d_w32 : h.d_w64,
-                             (unsigned)w.size(), h.d_counter, tile, h.d.fused, each, nblocks, g.stream);
+  return launch_matmult_list(h.d.T, h.d_items, h.d.items.data(), (int)h.d.items.size(), small ? h.d_w32 : h.d_w64,
+                             (unsigned)w.size(), small ? h.long32 : h.long64, h.d_counter, tile, h.d.fused, each, nblocks, g.stream);
 }
 
 // plan every entry through pdl_run_matmult's checks (outputs created as
@@ -1596,7 +1598,7 @@ static pdlhip_error list_build(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlhip_pdl
   // 8 bins, one per XCD (the kernels' list_next): each product, largest
   // inner dimension first, goes whole to the bin with the least work so far
   // (tiles x k); the bins lie back to back, bounds[x] .. bounds[x + 1]
-  auto build_work = [&](int tile, std::vector<int3> &work, unsigned *bounds) {
+  auto build_work = [&](int tile, std::vector<int3> &work, unsigned *bounds, unsigned &longest) {
     std::vector<std::vector<int3>> bins(8);
     std::vector<double> load(8, 0.0);
     for (int i : order) {
@@ -1611,14 +1613,15 @@ static pdlhip_error list_build(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlhip_pdl
     for (int x = 0; x < 8; x++) {
       bounds[x] = (unsigned)work.size();
       work.insert(work.end(), bins[x].begin(), bins[x].end());
+      longest = std::max(longest, (unsigned)bins[x].size());
     }
     bounds[8] = (unsigned)work.size();
   };
   // the device block: 8 bin counters 128 bytes apart, then the 64-tile
   // list's bounds, then the 32-tile list's
   unsigned qinit[256 + 9 + 9] = {0};
-  build_work(64, h.work64, qinit + 256);
-  build_work(32, h.work32, qinit + 265);
+  build_work(64, h.work64, qinit + 256, h.long64);
+  build_work(32, h.work32, qinit + 265, h.long32);
   // the matrix-core kernel indexes within a product with 32-bit offsets
   auto span = [](int64_t n1, int64_t i1, int64_t n2, int64_t i2) {
     return (n1 > 0 ? n1 - 1 : 0) * (i1 < 0 ? -i1 : i1) + (n2 > 0 ? n2 - 1 : 0) * (i2 < 0 ? -i2 : i2);
@@ -1640,17 +1643,17 @@ static pdlhip_error list_build(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlhip_pdl
   if (e == hipSuccess) e = upload_now(h.d_counter, qinit, sizeof qinit);
   if (e == hipSuccess) e = upload_now(h.d_w32, h.work32.data(), sizeof(int3) * h.work32.size());
   if (e == hipSuccess) e = upload_now(h.d_w64, h.work64.data(), sizeof(int3) * h.work64.size());
-  // tile by the autotuner: 32 / 64 SIMT tiles, the FP32/FP64 matrix-core
-  // kernel (0; 2: half the k per LDS stage) and, for float, the BF16
-  // three-way split (1); timed on a copy
-  // of the item table whose outputs all point into one scratch block
+  // tile by the autotuner: 32 / 64 SIMT tiles, the FP32/FP64 matrix cores
+  // with 64x64 (0) or 32x32 (2) work items and, for float, the BF16 three-way
+  // split (1); timed on a copy of the item table whose outputs all point into
+  // one scratch block
   if (e == hipSuccess) {
     std::vector<int> cands = {32, 64};
     if (h.mfma) { cands.push_back(0); cands.push_back(2); }
     if (h.mfma && h.d.T == PDLHIP_F) cands.push_back(1);
     const int dflt = h.mfma ? 0 : 64;
     char fam[160];
-    snprintf(fam, sizeof fam, "list:%s:mfma%d:fused%d:dim2^%d:items2^%d", type_name(h.d.T), h.mfma ? 1 : 0,
+    snprintf(fam, sizeof fam, "list:%s:tiles%d:fused%d:dim2^%d:items2^%d", type_name(h.d.T), h.mfma ? 1 : 0,
              h.d.fused ? 1 : 0, ilog2(maxdim), ilog2(nit));
     MmItem *t_items = nullptr;
     void *t_c = nullptr;

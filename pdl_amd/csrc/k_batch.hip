@@ -1,17 +1,19 @@
-// Lists of uneven matmults in one persistent launch (the reference runs
-// such a list as a Perl loop of matmult calls, lib/PDL/Primitive.pd:197-209
-// per item).  The host builds one work item per (product, C tile), ordered
-// by decreasing inner dimension (longest-processing-time first); persistent
-// blocks take items from a device counter until the queue is drained, so
-// every block reaches the exit condition.  Float and double lists in the
-// default modes run on the matrix cores (list_mfma_*); PDL order and the
-// integer types run the SIMT tile of k_matmult.hip (accumulation order per
-// output: ascending t, so the PDL-order variant stays bit-identical to PDL's
-// loop).
+// Lists of uneven matmults in one launch (the reference runs such a list as a
+// Perl loop of matmult calls, lib/PDL/Primitive.pd:197-209 per item).  The
+// host builds one work item per (product, C tile), ordered by decreasing
+// inner dimension (longest-processing-time first).  Float and double lists in
+// the default modes run on the matrix cores (list_tiles).  PDL order and the integer types run the SIMT tile of
+// k_matmult.hip (accumulation order per output: ascending t, so the PDL-order
+// variant stays bit-identical to PDL's loop) in persistent blocks, which take
+// items from a device counter until the queue is drained, so every block
+// reaches the exit condition; so does the BF16 split.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "device.hpp"
 #include "launch.hpp"
+#include "mm_tile.hpp"
 
 namespace pdlhip {
 
@@ -149,196 +151,264 @@ __global__ __launch_bounds__(256) void list_one(const MmItem *__restrict__ items
 
 // ---------------------------------------------------------------- matrix cores
 // Float and double lists in the default modes run on the matrix cores with
-// FP32 / FP64 products and sums (no operand scaling: the same arithmetic as
-// the FP32/FP64 SIMT kernel, summed in the matrix core's order): one work
-// item = a 64x64 tile of C, four waves of 32x32 each; a wave whose quadrant
-// lies outside the product skips its MFMAs.  k chunks (32 floats / 16
-// doubles) go global -> registers -> LDS ([k][row], [k][col]) with the next
-// chunk's loads in flight while the matrix cores work on the current one
-// (two LDS buffers, one barrier per chunk).
-//   float:  v_mfma_f32_32x32x2f32, lane l holds A[l%32][k + l/32] and
-//           B[k + l/32][l%32]; D reg r -> row 8(r/4) + 4(l/32) + r%4, col l%32
-//   double: v_mfma_f64_16x16x4f64 as 2x2 tiles, lane l holds A[l%16][k + l/16]
-//           and B[k + l/16][l%16]; D reg r -> row 4r + l/16, col l%16
-template <class T> struct ListMfma;
-template <> struct ListMfma<float> { static constexpr int KS = 32; };
-template <> struct ListMfma<double> { static constexpr int KS = 16; };
-
+// FP32 / FP64 products and sums: the instructions, stages and LDS rows of
+// mm_tile.hpp (float: partial sums of 32 k), TS x TS of C per work item.
+//
+// A tile lasts only a few stages, so a tile by itself is bound by the chain
+// it waits for: its work item, its operands' addresses, its first stages, one
+// memory latency each.  So a block runs through its work items as one
+// sequence of stages: two stages' loads are in flight while a third is
+// multiplied, also across the end of a tile.  Every fetch issues the same
+// loads whatever the tile's sizes (past the last stage, that stage again), so
+// that their waits stay counted: rows past an operand's last repeat it, and a
+// first stage of fewer k loads a whole one, or from the last k where that fits,
+// and is zeroed on its way to LDS.  A wave's 16x16 tiles lie 32 apart, so that where
+// no more than 32 rows or columns are inside the product each of the four
+// skips half of its instructions.
+//
+// Block b runs on XCD b % 8 and takes one item of each round of grid / 8 items
+// of bin b % 8, largest inner dimension first, so that the blocks' shares
+// differ little: the b / 8th of the first round and one five places on in each
+// next, lest a block meet the edge tiles of one product after the other.
+//
+// 4096 float products of 8..256 per side: 547 us (a tile at a time, taken from
+// a counter: 621; a workgroup per tile: 662), 63 TFLOP/s of the products' own
+// operations, 75 with the padding; double 937 (978).  300 of 8..64: 7.2 us
+// (14.5), 64 of 8..256: 14.9 (28.8), where the counter's latency was most of
+// it.  Four blocks per CU (without the partial sums) take as long as three,
+// and products of 256 alone reach 82 TFLOP/s: what is left is the LDS and
+// vector work between matrix instructions, about as long as those.
 typedef float lf32x16 __attribute__((ext_vector_type(16)));
-typedef double ld4 __attribute__((ext_vector_type(4)));
 
-template <class T, int KS>
-__device__ __forceinline__ void list_mfma_tile(const MmItem &it, int64_t tm, int64_t tn, T (*As)[KS][65],
-                                               T (*Bs)[KS][65]) {
-  constexpr int NE = KS / 4;            // staged elements per thread per operand (64 x KS / 256)
-  constexpr int SK = 256 / KS;          // rows apart of a thread's elements when it runs along k
-  // a product's own extent fits 32-bit offsets (checked by the host)
-  const T *a = (const T *)it.a + it.oa, *b = (const T *)it.b + it.ob;
-  T *c = (T *)it.c;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, wr = w >> 1, wc = w & 1;
-  const int H = (int)it.H, W = (int)it.W, K = (int)it.T;
-  const int h0 = (int)tm * 64, w0 = (int)tn * 64;
-  const int a_t = (int)it.a_t, a_h = (int)it.a_h, b_w = (int)it.b_w, b_t = (int)it.b_t;
-  // threads run along whichever index of each operand is unit-stride: a
-  // thread keeps one "fast" index (k, or the row/column) and steps the other
-  const bool a_kfast = a_t == 1 || a_h != 1;
-  const bool b_wfast = b_w == 1 || b_t != 1;
-  const int fa = a_kfast ? tid % KS : tid % 64, sa = a_kfast ? tid / KS : tid / 64, da = a_kfast ? SK : 4;
-  const int fb = b_wfast ? tid % 64 : tid % KS, sb = b_wfast ? tid / 64 : tid / KS, db = b_wfast ? 4 : SK;
-  const bool active = h0 + 32 * wr < H && w0 + 32 * wc < W;
-  // a chunk wholly inside both operands loads without clamps or masks: one
-  // base address per operand, the thread's elements a constant stride apart
-  const bool inside_hw = h0 + 64 <= H && w0 + 64 <= W;
-  const int a_step = da * (a_kfast ? a_h : a_t), b_step = db * (b_wfast ? b_t : b_w);
-  T ra[NE], rb[NE];
-  // edge chunks: loads clamped into the operand (the element is zeroed when
-  // staged), so no load sits behind a branch
-  auto load = [&](int k0) {
-    if (inside_hw && k0 + KS <= K) {
-      const T *pa = a + (a_kfast ? (k0 + fa) * a_t + (h0 + sa) * a_h : (k0 + sa) * a_t + (h0 + fa) * a_h);
-      const T *pb = b + (b_wfast ? (w0 + fb) * b_w + (k0 + sb) * b_t : (w0 + sb) * b_w + (k0 + fb) * b_t);
+template <int TS> constexpr int LIST_PER_CU = TS == 32 ? 6 : 3;
+
+// one operand's loads: thread t takes group % 8 of row / 8 (KFAST) or row t %
+// TS, as TileLoad does
+template <class T, int TS, bool KFAST> struct ListLoad {
+  static constexpr int P = TS * 8 / 256, V = TILE_V<T>, KB = TILE_K<T>;
+  typedef typename TileType<T>::vec_t vec;
+  typedef vec __attribute__((aligned(sizeof(T)))) vecu;
+  gptr<const T> at[P];   // the thread's k of the stage
+  int64_t inc_k;
+  vec v[2][P];
+  __device__ static int row(int s) { const int e = threadIdx.x + 256 * s; return KFAST ? e / 8 : e % TS; }
+  __device__ static int group(int s) { const int e = threadIdx.x + 256 * s; return KFAST ? e % 8 : e / TS; }
+  // `top`: the last k at which V of them can be loaded (KB: anywhere in a stage)
+  __device__ __forceinline__ void open(const T *base, int r0, int R, int64_t inc_r, int64_t ik, int top) {
 #pragma unroll
-      for (int q = 0; q < NE; q++) {
-        ra[q] = pa[q * a_step];
-        rb[q] = pb[q * b_step];
-      }
-      return;
+    for (int s = 0; s < P; s++) {
+      const int r = r0 + row(s) < R ? r0 + row(s) : R - 1;
+      const int k = V * group(s);
+      at[s] = as_global(base + r * inc_r + (k < top ? k : top) * ik);
     }
+    inc_k = ik;
+  }
+  // a stage's loads; `most`: the last of the V that there is (strided only)
+  __device__ __forceinline__ void load(int set, int most) {
 #pragma unroll
-    for (int q = 0; q < NE; q++) {
-      const int s1 = sa + da * q, s2 = sb + db * q;
-      const int ah = a_kfast ? h0 + s1 : h0 + fa, ak = a_kfast ? k0 + fa : k0 + s1;
-      const int bw = b_wfast ? w0 + fb : w0 + s2, bk = b_wfast ? k0 + s2 : k0 + fb;
-      ra[q] = a[(ak < K ? ak : K - 1) * a_t + (ah < H ? ah : H - 1) * a_h];
-      rb[q] = b[(bw < W ? bw : W - 1) * b_w + (bk < K ? bk : K - 1) * b_t];
-    }
-  };
-  // interior chunks of the common layout (a's k and b's w unit-stride):
-  // every staged element lands at a slot a compile-time distance from the
-  // thread's first, with no bounds tests
-  const bool plain = a_t == 1 && b_w == 1;
-  auto stage = [&](int buf, int k0) {
-    const bool inside = inside_hw && k0 + KS <= K;
-    if (plain && inside) {
+    for (int s = 0; s < P; s++) {
+      if (KFAST) v[set][s] = *(gptr<const vecu>)at[s];
+      else
 #pragma unroll
-      for (int q = 0; q < NE; q++) {
-        As[buf][fa][sa + SK * q] = ra[q];
-        Bs[buf][sb + 4 * q][fb] = rb[q];
-      }
-      return;
-    }
-#pragma unroll
-    for (int q = 0; q < NE; q++) {
-      const int s1 = sa + da * q, s2 = sb + db * q;
-      const int mm = a_kfast ? s1 : fa, kk = a_kfast ? fa : s1;
-      const int nn = b_wfast ? fb : s2, kb = b_wfast ? s2 : fb;
-      As[buf][kk][mm] = (inside || (h0 + mm < H && k0 + kk < K)) ? ra[q] : T(0);
-      Bs[buf][kb][nn] = (inside || (w0 + nn < W && k0 + kb < K)) ? rb[q] : T(0);
-    }
-  };
-  if constexpr (sizeof(T) == 4) {
-    lf32x16 acc;
-#pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = 0.0f;
-    // an empty inner dimension loads nothing (its clamp would reach index
-    // -1) and stores the zero sums
-    if (K > 0) load(0);
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += KS) {
-      stage(buf, k0);
-      __syncthreads();
-      if (k0 + KS < K) load(k0 + KS);
-      // every wave multiplies, also one whose quarter lies outside the
-      // product (its LDS rows are zeros and it stores nothing): a branch
-      // here makes the compiler copy the accumulators out of AGPRs and back
-      // each chunk
-#pragma unroll
-      for (int kk = 0; kk < KS; kk += 2) {
-        const float av = As[buf][kk + (lane >> 5)][32 * wr + (lane & 31)];
-        const float bv = Bs[buf][kk + (lane >> 5)][32 * wc + (lane & 31)];
-        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
-      }
-      buf ^= 1;
-    }
-    if (active) {
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int64_t gh = h0 + 32 * wr + 8 * (r / 4) + 4 * (lane >> 5) + (r & 3);
-        const int64_t gw = w0 + 32 * wc + (lane & 31);
-        if (gh < H && gw < W) c[it.oc + gw * it.c_w + gh * it.c_h] = acc[r];
-      }
-    }
-  } else {
-    ld4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-      for (int j = 0; j < 2; j++) acc[i][j] = ld4{0.0, 0.0, 0.0, 0.0};
-    // an empty inner dimension loads nothing (its clamp would reach index
-    // -1) and stores the zero sums
-    if (K > 0) load(0);
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += KS) {
-      stage(buf, k0);
-      __syncthreads();
-      if (k0 + KS < K) load(k0 + KS);
-#pragma unroll
-      for (int kk = 0; kk < KS; kk += 4) {
-        double af[2], bf[2];
-#pragma unroll
-        for (int i = 0; i < 2; i++) af[i] = As[buf][kk + (lane >> 4)][32 * wr + 16 * i + (lane & 15)];
-#pragma unroll
-        for (int j = 0; j < 2; j++) bf[j] = Bs[buf][kk + (lane >> 4)][32 * wc + 16 * j + (lane & 15)];
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-          for (int j = 0; j < 2; j++)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(af[i], bf[j], acc[i][j], 0, 0, 0);
-      }
-      buf ^= 1;
-    }
-    if (active) {
-#pragma unroll
-      for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-          for (int r = 0; r < 4; r++) {
-            const int64_t gh = h0 + 32 * wr + 16 * i + 4 * r + (lane >> 4);
-            const int64_t gw = w0 + 32 * wc + 16 * j + (lane & 15);
-            if (gh < H && gw < W) c[it.oc + gw * it.c_w + gh * it.c_h] = acc[i][j][r];
-          }
+        for (int i = 0; i < V; i++) v[set][s][i] = at[s][(i < most ? i : most) * inc_k];
     }
   }
-  // the LDS buffers are refilled by the next work item
+  __device__ __forceinline__ void advance(int k) {
+#pragma unroll
+    for (int s = 0; s < P; s++) at[s] += k * inc_k;
+  }
+  // zero from `some` k on; what was loaded from `top` instead of the group's
+  // own k goes back to its place
+  __device__ __forceinline__ void stage(int set, int some, int top, T (*l)[TILE_P<T>]) {
+    if (some < KB) {
+#pragma unroll
+      for (int s = 0; s < P; s++) {
+        const int k = V * group(s), d = k < top ? 0 : k - top;
+        vec x;
+#pragma unroll
+        for (int i = 0; i < V; i++) {
+          x[i] = T(0);
+#pragma unroll
+          for (int j = i; j < V; j++) x[i] = d == j - i ? v[set][s][j] : x[i];
+          x[i] = i < some - k ? x[i] : T(0);
+        }
+        v[set][s] = x;
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < P; s++) *reinterpret_cast<vec *>(&l[row(s)][V * group(s)]) = v[set][s];
+  }
+};
+
+// `work` null: the tiles of product `only`, ntn of them a row, one a block
+template <class T, int TS, bool AK, bool BK>
+__global__ __launch_bounds__(256, LIST_PER_CU<TS>) void list_tiles(const MmItem *__restrict__ items,
+                                                                    const int3 *__restrict__ work,
+                                                                    const unsigned int *__restrict__ bounds, int only,
+                                                                    unsigned ntn) {
+  constexpr int KB = TILE_K<T>, V = TILE_V<T>, TI = TS / 32;
+  // of a stage: ends its tile; more than 32 rows, columns of it inside the
+  // product; more than half of its k
+  constexpr unsigned LAST = 1, HIGH = 2, WIDE = 4, DEEP = 8, KIND = 4;
+  typedef TileType<T> TT;
+  __shared__ __align__(16) T sA[2][TS][TILE_P<T>];
+  __shared__ __align__(16) T sB[2][TS][TILE_P<T>];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int wr = w >> 1, wc = w & 1, fr = lane & 15, fk = lane >> 4;
+  const unsigned bin = blockIdx.x % LIST_BINS, step = work ? gridDim.x / LIST_BINS : gridDim.x;
+  const unsigned end = work ? bounds[bin + 1] : gridDim.x, turn = 5 % step;
+  struct Place {
+    unsigned round, slot;
+    __device__ unsigned at() const { return round + slot; }
+  };
+  auto after = [&](Place p) {
+    const unsigned slot = p.slot + turn;
+    return Place{p.round + step, slot < step ? slot : slot - step};
+  };
+  Place lw = {work ? bounds[bin] : 0, work ? blockIdx.x / LIST_BINS : blockIdx.x}, cw = lw;   // loaded, multiplied item
+  if (lw.at() >= end) return;
+  auto job_at = [&](unsigned i) { return work ? work[i] : make_int3(only, (int)(i / ntn), (int)(i % ntn)); };
+  ListLoad<T, TS, AK> la;
+  ListLoad<T, TS, BK> lb;
+  // the loaded item: stages left, the first one's k, HIGH and WIDE, and for
+  // its loads: the last k for a whole group, the last of a group's k
+  int left = 0, first = 0, top = 0, most = 0;
+  unsigned sides = 0;
+  auto open = [&]() {
+    const int3 job = job_at(lw.at());
+    const MmItem &it = items[job.x];
+    const int K = (int)it.T;
+    const bool any = K > 0;   // an empty inner dimension: one stage of zeros, its loads from the item table
+    left = any ? (K - 1) / KB + 1 : 1;
+    first = any ? (K - 1) % KB + 1 : 0;
+    top = K >= KB ? KB : K > V ? K - V : 0;
+    most = K >= V ? V - 1 : any ? K - 1 : 0;
+    la.open(any ? (const T *)it.a + it.oa : (const T *)items, any ? job.y * TS : 0, any ? (int)it.H : 1,
+            it.a_h, any ? it.a_t : 0, top);
+    lb.open(any ? (const T *)it.b + it.ob : (const T *)items, any ? job.z * TS : 0, any ? (int)it.W : 1,
+            it.b_w, any ? it.b_t : 0, top);
+    sides = ((int)it.H - job.y * TS > 32 ? HIGH : 0) | ((int)it.W - job.z * TS > 32 ? WIDE : 0);
+  };
+  int some[2], tops[2];   // of the stages in the two register sets
+  unsigned kinds = 0;     // of the stages ahead, KIND bits each
+  int ahead = 0;
+  bool fresh = true;
+  auto fetch = [&](int set) {
+    if (left == 0 && after(lw).at() < end) {
+      lw = after(lw);
+      open();
+      fresh = true;
+    }
+    la.load(set, most);
+    lb.load(set, most);
+    some[set] = fresh ? first : KB;
+    tops[set] = top;
+    kinds |= (sides | (left == 1 ? LAST : 0) | (some[set] > KB / 2 ? DEEP : 0)) << (KIND * ahead);
+    const int go = left > 1 ? some[set] : 0;
+    la.advance(go);
+    lb.advance(go);
+    fresh = false;
+    if (left > 0) left--;
+  };
+  typename TT::acc_t acc[TI][TI], part[TI][TI];
+  typename TT::vec_t af[2][TI], bf[2][TI];
+  auto clear = [&]() {
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+      for (int j = 0; j < TI; j++) acc[i][j] = part[i][j] = typename TT::acc_t{T(0), T(0), T(0), T(0)};
+  };
+  auto frags = [&](int half, int buf) {
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+      af[half][i] = *reinterpret_cast<const typename TT::vec_t *>(&sA[buf][(2 * i + wr) * 16 + fr][half * KB / 2 + V * fk]);
+#pragma unroll
+    for (int j = 0; j < TI; j++)
+      bf[half][j] = *reinterpret_cast<const typename TT::vec_t *>(&sB[buf][(2 * j + wc) * 16 + fr][half * KB / 2 + V * fk]);
+  };
+  auto mult = [&](int half, int ni, int nj) {
+#pragma unroll
+    for (int u = 0; u < V; u++)
+#pragma unroll
+      for (int i = 0; i < ni; i++)
+#pragma unroll
+        for (int j = 0; j < nj; j++) {
+          if constexpr (sizeof(T) == 8) {
+            acc[i][j] = TT::mfma(af[half][i][u], bf[half][j][u], acc[i][j]);
+          } else {
+            if (half == 0 && u == 0) acc[i][j] += part[i][j];
+            part[i][j] = TT::mfma(af[half][i][u], bf[half][j][u], half == 0 && u == 0 ? typename TT::acc_t{} : part[i][j]);
+          }
+        }
+  };
+  auto multiply = [&](int half) {
+    if (half == 1 && !(kinds & DEEP)) return;
+    if constexpr (TI == 1) {
+      mult(half, 1, 1);
+    } else if (kinds & HIGH) {
+      if (kinds & WIDE) mult(half, 2, 2);
+      else mult(half, 2, 1);
+    } else {
+      if (kinds & WIDE) mult(half, 1, 2);
+      else mult(half, 1, 1);
+    }
+  };
+  auto store = [&]() {
+    const int3 job = job_at(cw.at());
+    const MmItem &it = items[job.x];
+    const int64_t m0 = (int64_t)job.y * TS, n0 = (int64_t)job.z * TS, c_h = it.c_h, c_w = it.c_w;
+    const int rows = (int)(it.H - m0 < TS ? it.H - m0 : TS), cols = (int)(it.W - n0 < TS ? it.W - n0 : TS);
+    const auto c = as_global((T *)it.c + it.oc + m0 * c_h + n0 * c_w);
+#pragma unroll
+    for (int i = 0; i < TI; i++)
+#pragma unroll
+      for (int j = 0; j < TI; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int h = (2 * i + wr) * 16 + TT::row(r, fk), n = (2 * j + wc) * 16 + fr;
+          T v = acc[i][j][r];
+          if constexpr (sizeof(T) == 4) v += part[i][j][r];
+          if (h < rows && n < cols) c[h * c_h + n * c_w] = v;
+        }
+  };
+  // multiplies the stage in buffer cur (the order of tile_product's step)
+  auto run = [&](int cur) {
+    la.stage(cur ^ 1, some[cur ^ 1], tops[cur ^ 1], sA[cur ^ 1]);
+    lb.stage(cur ^ 1, some[cur ^ 1], tops[cur ^ 1], sB[cur ^ 1]);
+    fetch(cur ^ 1);
+    frags(1, cur);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(0);
+    __syncthreads();
+    frags(0, cur ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(1);
+    const bool last = kinds & LAST;
+    kinds >>= KIND;
+    if (last) {
+      store();
+      cw = after(cw);
+      clear();
+    }
+  };
+  clear();
+  open();
+  fetch(0);
+  ahead = 1;
+  fetch(1);
+  la.stage(0, some[0], tops[0], sA[0]);
+  lb.stage(0, some[0], tops[0], sB[0]);
+  ahead = 2;
+  fetch(0);
+  ahead = 3;
   __syncthreads();
-}
-
-// KS: k per LDS stage (the type's default, or half of it: half the LDS per
-// block, more resident blocks to cover load latency); the register budget
-// matches what the LDS allows (4 blocks of 4 waves per CU at the default
-// stage, 6 at half)
-template <class T, int KS>
-__global__ __launch_bounds__(256, KS == ListMfma<T>::KS ? 4 : 6) void list_mfma_queue(const MmItem *__restrict__ items,
-                                                       const int3 *__restrict__ work,
-                                                       const unsigned int *__restrict__ bounds,
-                                                       unsigned int *counter) {
-  __shared__ T As[2][KS][65];
-  __shared__ T Bs[2][KS][65];
-  __shared__ unsigned int next;
-  int bin = blockIdx.x % LIST_BINS;
-  unsigned done = 0;
-  int3 job;
-  while (list_next(counter, bounds, work, bin, done, &next, job))
-    list_mfma_tile<T, KS>(items[job.x], job.y, job.z, As, Bs);
-}
-
-template <class T, int KS>
-__global__ __launch_bounds__(256, KS == ListMfma<T>::KS ? 4 : 6) void list_mfma_one(const MmItem *__restrict__ items,
-                                                                                   int idx, int64_t ntn) {
-  __shared__ T As[2][KS][65];
-  __shared__ T Bs[2][KS][65];
-  list_mfma_tile<T, KS>(items[idx], blockIdx.x / ntn, blockIdx.x % ntn, As, Bs);
+  frags(0, 0);
+  // (a stage past the last one ends no tile; leaving between the two would
+  // make the waits at the top of the loop count that path's loads)
+  do {
+    run(0);
+    run(1);
+  } while (cw.at() < end);
 }
 
 // ---------------------------------------------------------------- float on BF16 matrix cores
@@ -443,7 +513,8 @@ __device__ __forceinline__ void list_bf16x3_tile(const MmItem &it, int64_t tm, i
     stage(buf, k0);
     __syncthreads();
     if (k0 + BKS < K) load(k0 + BKS);
-    {   // every wave multiplies (see list_mfma_tile)
+    {   // every wave multiplies (a branch here makes the
+        // compiler copy the accumulators out of AGPRs and back each chunk)
 #pragma unroll
       for (int ks = 0; ks < 2; ks++) {
         const int sa = (ks * 2 + fseg) ^ ((ar_ >> 1) & 3), sb = (ks * 2 + fseg) ^ ((br_ >> 1) & 3);
@@ -509,19 +580,36 @@ static hipError_t list_bf16x3(const MmItem *d_items, const MmItem *h_items, int 
   return hipGetLastError();
 }
 
-template <class T, int KS>
-static hipError_t list_mfma_T(const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
-                              unsigned int nwork, unsigned int *d_counter, bool each, int nblocks, hipStream_t s) {
-  if (!each) {
-    hipLaunchKernelGGL(list_reset, dim3(1), dim3(64), 0, s, d_counter);
-    hipLaunchKernelGGL((list_mfma_queue<T, KS>), dim3(nblocks), dim3(256), 0, s, d_items, d_work,
-                       (const unsigned int *)d_counter + LIST_BOUNDS, d_counter);
+template <class T, int TS>
+static hipError_t list_tiles_T(const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
+                               unsigned longest, unsigned int *d_counter, bool each, hipStream_t s) {
+  // 16-byte loads along k where every product has it unit-stride and as many
+  // k as one load takes
+  bool ak = true, bk = true;
+  for (int i = 0; i < nitems; i++) {
+    const bool whole = h_items[i].T >= TILE_V<T> || h_items[i].T == 0;
+    ak = ak && h_items[i].a_t == 1 && whole;
+    bk = bk && h_items[i].b_t == 1 && whole;
+  }
+  auto go = [&](unsigned grid, const int3 *work, int only, unsigned ntn) {
+    const unsigned int *bounds = (const unsigned int *)d_counter + LIST_BOUNDS + (TS == 32 ? LIST_BINS + 1 : 0);
+    if (ak && bk)
+      hipLaunchKernelGGL((list_tiles<T, TS, true, true>), dim3(grid), dim3(256), 0, s, d_items, work, bounds, only, ntn);
+    else if (ak)
+      hipLaunchKernelGGL((list_tiles<T, TS, true, false>), dim3(grid), dim3(256), 0, s, d_items, work, bounds, only, ntn);
+    else if (bk)
+      hipLaunchKernelGGL((list_tiles<T, TS, false, true>), dim3(grid), dim3(256), 0, s, d_items, work, bounds, only, ntn);
+    else
+      hipLaunchKernelGGL((list_tiles<T, TS, false, false>), dim3(grid), dim3(256), 0, s, d_items, work, bounds, only, ntn);
+  };
+  if (!each) {   // as many blocks as are resident at once
+    go(LIST_BINS * std::min(std::max(longest, 1u), 32u * LIST_PER_CU<TS>), d_work, 0, 1);
     return hipGetLastError();
   }
   for (int i = 0; i < nitems; i++) {
-    const int64_t ntm = (h_items[i].H + 63) / 64, ntn = (h_items[i].W + 63) / 64;
+    const int64_t ntm = (h_items[i].H + TS - 1) / TS, ntn = (h_items[i].W + TS - 1) / TS;
     if (ntm * ntn == 0) continue;             // an empty k stores zeros
-    hipLaunchKernelGGL((list_mfma_one<T, KS>), dim3((unsigned)(ntm * ntn)), dim3(256), 0, s, d_items, i, ntn);
+    go((unsigned)(ntm * ntn), nullptr, i, (unsigned)ntn);
   }
   return hipGetLastError();
 }
@@ -552,24 +640,21 @@ static hipError_t list_T(const MmItem *d_items, const MmItem *h_items, int nitem
 }
 
 hipError_t launch_matmult_list(int T, const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
-                               unsigned int nwork, unsigned int *d_counter, int tile, bool fused, bool each,
-                               int nblocks, hipStream_t s) {
-  // tile 0: the matrix-core kernels (64x64 work items), float/double lists
-  // in the default modes; tile 1: float on the BF16 matrix cores
+                               unsigned int nwork, unsigned int longest, unsigned int *d_counter, int tile, bool fused,
+                               bool each, int nblocks, hipStream_t s) {
+  // tile 0 / 2: the matrix-core kernels (64x64 / 32x32 work items), float and
+  // double lists in the default modes; tile 1: float on the BF16 matrix cores
   if (tile == 1 && fused && T == PDLHIP_F)
     return list_bf16x3(d_items, h_items, nitems, d_work, nwork, d_counter, each, nblocks, s);
   if (tile == 1) tile = 0;
-  constexpr int KF = ListMfma<float>::KS, KD = ListMfma<double>::KS;
-  if (tile == 2 && fused && T == PDLHIP_F)
-    return list_mfma_T<float, KF / 2>(d_items, h_items, nitems, d_work, nwork, d_counter, each, nblocks, s);
-  if (tile == 2 && fused && T == PDLHIP_D)
-    return list_mfma_T<double, KD / 2>(d_items, h_items, nitems, d_work, nwork, d_counter, each, nblocks, s);
-  if (tile == 2) tile = 0;
-  if (tile == 0 && fused && T == PDLHIP_F)
-    return list_mfma_T<float, KF>(d_items, h_items, nitems, d_work, nwork, d_counter, each, nblocks, s);
-  if (tile == 0 && fused && T == PDLHIP_D)
-    return list_mfma_T<double, KD>(d_items, h_items, nitems, d_work, nwork, d_counter, each, nblocks, s);
+  if (fused && T == PDLHIP_F && (tile == 0 || tile == 2))
+    return tile == 0 ? list_tiles_T<float, 64>(d_items, h_items, nitems, d_work, longest, d_counter, each, s)
+                     : list_tiles_T<float, 32>(d_items, h_items, nitems, d_work, longest, d_counter, each, s);
+  if (fused && T == PDLHIP_D && (tile == 0 || tile == 2))
+    return tile == 0 ? list_tiles_T<double, 64>(d_items, h_items, nitems, d_work, longest, d_counter, each, s)
+                     : list_tiles_T<double, 32>(d_items, h_items, nitems, d_work, longest, d_counter, each, s);
   if (tile == 0) tile = 64;
+  if (tile == 2) tile = 32;
   switch (T) {
 #define X(TC) case TC: return list_T<CType<TC>::T>(d_items, h_items, nitems, d_work, nwork, d_counter, tile, \
                                                    fused, each, nblocks, s);

@@ -29,10 +29,10 @@ PDLHIP_FOR_EACH_TYPE(X)
 PDLHIP_FOR_EACH_TYPE(X)
 #undef X
 
-// a list of products in one persistent work-queue launch, or one launch per
-// product (each = true) (k_batch.hip)
+// a list of products in one persistent launch, or one launch per product
+// (each = true) (k_batch.hip); longest: work items of the longest of 8 bins
 hipError_t launch_matmult_list(int T, const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
-                               unsigned int nwork, unsigned int *d_counter, int tile, bool fused, bool each,
+                               unsigned int nwork, unsigned int longest, unsigned int *d_counter, int tile, bool fused, bool each,
                                int nblocks, hipStream_t s);
 
 // Bad.pd elementwise ops (k_badops.hip): a of type T, mask int32 (setbadif),
