@@ -1704,7 +1704,7 @@ struct RaggedH {
   bool scan = false;
   int T = -1, op = -1, n = 0;
   RagLaunch L;
-  void *d_items = nullptr, *d_segs = nullptr, *d_multi = nullptr, *d_order = nullptr, *d_bstart = nullptr,
+  void *d_items = nullptr, *d_segs = nullptr, *d_multi = nullptr, *d_pieces = nullptr, *d_bstart = nullptr,
        *d_scratch = nullptr, *d_empty = nullptr;
 };
 
@@ -1855,32 +1855,60 @@ static pdlhip_error ragged_finish(const char *who, RaggedH &h, std::vector<RagIt
     for (int k = 0; k < h.L.prog.nin; k++)
       if (it.inc[k]) bytes += (size_t)it.len * type_size(h.L.prog.type[k]);
   h.L.prog.stream = streaming_read(bytes) ? 1 : 0;
+  // reductions: a wave takes a segment, whose steps it waits for one by one;
+  // shorter segments (down to the 512 elements of one step) where 4096-element
+  // ones would leave fewer than 16 waves per CU (2e6 elements in 233 vectors:
+  // 32 us at 4096, 15 at 512)
+  int64_t total = 0;
+  for (const RagItem &it : items) total += it.len;
+  int64_t seglen = RAG_SEG;
+  while (!h.scan && seglen > 512 && total / seglen < 4096) seglen /= 2;
   std::vector<RagSeg> segs;
   std::vector<int32_t> multi;
   for (int i = 0; i < n; i++) {
     RagItem &it = items[i];
     it.seg0 = (int64_t)segs.size();
-    it.nseg = std::max<int64_t>(1, (it.len + RAG_SEG - 1) / RAG_SEG);
+    it.nseg = std::max<int64_t>(1, (it.len + seglen - 1) / seglen);
     for (int64_t k = 0; k < it.nseg; k++) {
       RagSeg sg;
       sg.item = i;
       sg.single = it.nseg == 1;
-      sg.start = k * RAG_SEG;
-      sg.end = std::min<int64_t>(it.len, (k + 1) * RAG_SEG);
+      sg.start = k * seglen;
+      sg.end = std::min<int64_t>(it.len, (k + 1) * seglen);
       segs.push_back(sg);
     }
-    if (it.nseg > 1 && h.op != RAG_NOREDUCE) multi.push_back(i);
+    if (it.nseg > 1 && h.op != RAG_NOREDUCE && !h.scan) multi.push_back(i);
   }
   h.L.nseg = (int64_t)segs.size();
-  h.L.nmulti = (int64_t)multi.size();
   // scans: items to blocks longest-first onto the least loaded block (LPT);
-  // each block then runs its items longest-first
-  std::vector<int32_t> order, bstart;
+  // each block then runs its items longest-first.  The longest item bounds
+  // that, so items longer than 5/4 of a block's mean share are cut into pieces
+  // of about that share, which start from the totals of the segments before
+  // them: those segments are read twice.  40000 vectors of lognormal lengths,
+  // 3.6e8 elements, 4% of them twice: 17 + 1320 us (uncut: 1550, the longest
+  // vector three shares); 233, 2e6 elements, 77% twice, from the caches: 7 + 10
+  // us (70, 13 shares)
+  std::vector<RagPiece> pieces;
+  std::vector<int32_t> bstart;
   if (h.scan) {
-    const int nblk = std::min(n, 1024);
-    std::vector<int32_t> byl(n);
-    for (int i = 0; i < n; i++) byl[i] = i;
-    std::stable_sort(byl.begin(), byl.end(), [&](int32_t x, int32_t y) { return items[x].len > items[y].len; });
+    const int64_t share = ((total + 1023) / 1024 + RAG_SEG - 1) / RAG_SEG * RAG_SEG;
+    std::vector<RagPiece> all;
+    for (int i = 0; i < n; i++) {
+      const RagItem &it = items[i];
+      const int64_t np = it.len > share + share / 4 ? (it.len + share - 1) / share : 1;
+      const int64_t step = np == 1 ? it.len : ((it.len + np - 1) / np + RAG_SEG - 1) / RAG_SEG * RAG_SEG;
+      for (int64_t c = 0; c == 0 || c < it.len; c += step) {
+        if (c > 0)
+          for (int64_t k = (c - step) / RAG_SEG; k < c / RAG_SEG; k++) multi.push_back((int32_t)(it.seg0 + k));
+        all.push_back(RagPiece{c, std::min(it.len, c + step), i, 0});
+        if (step == 0) break;
+      }
+    }
+    const int np = (int)all.size(), nblk = std::min(np, 1024);
+    std::vector<int32_t> byl(np);
+    for (int i = 0; i < np; i++) byl[i] = i;
+    auto len = [&](int32_t i) { return all[i].end - all[i].start; };
+    std::stable_sort(byl.begin(), byl.end(), [&](int32_t x, int32_t y) { return len(x) > len(y); });
     std::vector<std::vector<int32_t>> bins(nblk);
     std::priority_queue<std::pair<int64_t, int32_t>, std::vector<std::pair<int64_t, int32_t>>,
                         std::greater<std::pair<int64_t, int32_t>>> pq;
@@ -1889,15 +1917,16 @@ static pdlhip_error ragged_finish(const char *who, RaggedH &h, std::vector<RagIt
       auto top = pq.top();
       pq.pop();
       bins[top.second].push_back(i);
-      pq.push({top.first + items[i].len + 256, top.second});   // + per-item overhead
+      pq.push({top.first + len(i) + 256, top.second});   // + per-piece overhead
     }
     bstart.push_back(0);
     for (auto &bn : bins) {
-      order.insert(order.end(), bn.begin(), bn.end());
-      bstart.push_back((int32_t)order.size());
+      for (int32_t i : bn) pieces.push_back(all[i]);
+      bstart.push_back((int32_t)pieces.size());
     }
     h.L.nblk = nblk;
   }
+  h.L.nmulti = (int64_t)multi.size();
   if (g.plan_only) { *hout = new RaggedH(h); return ok(); }
   auto up = [&](const void *src, size_t bytes, void **dst) -> bool {
     *dst = dev_alloc(std::max<size_t>(bytes, 1));
@@ -1907,19 +1936,19 @@ static pdlhip_error ragged_finish(const char *who, RaggedH &h, std::vector<RagIt
   bool okk = up(items.data(), sizeof(RagItem) * items.size(), &h.d_items) &&
              up(segs.data(), sizeof(RagSeg) * segs.size(), &h.d_segs) &&
              up(multi.data(), sizeof(int32_t) * multi.size(), &h.d_multi) &&
-             up(order.data(), sizeof(int32_t) * order.size(), &h.d_order) &&
+             up(pieces.data(), sizeof(RagPiece) * pieces.size(), &h.d_pieces) &&
              up(bstart.data(), sizeof(int32_t) * bstart.size(), &h.d_bstart);
   h.d_scratch = dev_alloc(std::max<size_t>(64 * segs.size(), 64));
   h.d_empty = dev_alloc(std::max<size_t>(sizeof(int32_t) * n, 4));
   if (!okk || !h.d_scratch || !h.d_empty) {
-    for (void *p : {h.d_items, h.d_segs, h.d_multi, h.d_order, h.d_bstart, h.d_scratch, h.d_empty}) dev_free(p);
+    for (void *p : {h.d_items, h.d_segs, h.d_multi, h.d_pieces, h.d_bstart, h.d_scratch, h.d_empty}) dev_free(p);
     return oom_err(who);
   }
   h.L.empty = (int32_t *)h.d_empty;
   h.L.items = (const RagItem *)h.d_items;
   h.L.segs = (const RagSeg *)h.d_segs;
   h.L.multi = (const int32_t *)h.d_multi;
-  h.L.order = (const int32_t *)h.d_order;
+  h.L.pieces = (const RagPiece *)h.d_pieces;
   h.L.bstart = (const int32_t *)h.d_bstart;
   h.L.scratch = h.d_scratch;
   *hout = new RaggedH(h);
@@ -2670,7 +2699,7 @@ pdlhip_error pdlhip_ragged_count(pdlhip_ragged *handle, int64_t *nitems) {
 pdlhip_error pdlhip_ragged_free(pdlhip_ragged *handle) {
   if (!handle) return ok();
   RaggedH &h = handle->h;
-  for (void *p : {h.d_items, h.d_segs, h.d_multi, h.d_order, h.d_bstart, h.d_scratch, h.d_empty}) dev_free(p);
+  for (void *p : {h.d_items, h.d_segs, h.d_multi, h.d_pieces, h.d_bstart, h.d_scratch, h.d_empty}) dev_free(p);
   delete handle;
   return ok();
 }

@@ -125,6 +125,7 @@ struct RagItem {
   int64_t len, seg0, nseg;
 };
 struct RagSeg { int32_t item, single; int64_t start, end; };
+struct RagPiece { int64_t start, end; int32_t item, pad; };   // start: a multiple of RAG_SEG
 struct RagLaunch {
   RagProg prog;
   const RagItem *items;
@@ -136,8 +137,10 @@ struct RagLaunch {
   int64_t nmulti;
   void *scratch;                // 64 bytes per segment
   int32_t *empty;               // minimum/maximum: per item, 1 when no good value was found
-  // scans: one block per item; block b runs items order[bstart[b] .. bstart[b+1])
-  const int32_t *order;
+  // scans: block b runs pieces[bstart[b] .. bstart[b+1]); `multi` lists the
+  // segments that lie before an item's last piece, whose totals go to scratch
+  // (8 bytes per segment)
+  const RagPiece *pieces;
   const int32_t *bstart;
   int32_t nblk;
 };
