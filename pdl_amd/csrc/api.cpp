@@ -1858,11 +1858,16 @@ static pdlhip_error ragged_finish(const char *who, RaggedH &h, std::vector<RagIt
   // reductions: a wave takes a segment, whose steps it waits for one by one;
   // shorter segments (down to the 512 elements of one step) where 4096-element
   // ones would leave fewer than 16 waves per CU (2e6 elements in 233 vectors:
-  // 32 us at 4096, 15 at 512)
-  int64_t total = 0;
-  for (const RagItem &it : items) total += it.len;
+  // 32 us at 4096, 15 at 512).  Not where no item is longer than one segment:
+  // that would add the combine's launch (2048 rows of 2048 doubles 39 us
+  // instead of 35)
+  int64_t total = 0, longest = 0;
+  for (const RagItem &it : items) {
+    total += it.len;
+    longest = std::max(longest, it.len);
+  }
   int64_t seglen = RAG_SEG;
-  while (!h.scan && seglen > 512 && total / seglen < 4096) seglen /= 2;
+  while (!h.scan && longest > RAG_SEG && seglen > 512 && total / seglen < 4096) seglen /= 2;
   std::vector<RagSeg> segs;
   std::vector<int32_t> multi;
   for (int i = 0; i < n; i++) {
