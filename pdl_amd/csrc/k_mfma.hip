@@ -34,6 +34,8 @@
 // block tile and K to the k step (zeros).
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "device.hpp"
 #include "launch.hpp"
 #include "mfma_common.hpp"
@@ -457,10 +459,14 @@ __device__ __forceinline__ float pdl_dot_f32(const float *a, int64_t at, const f
 // row's columns are re-tested with mm_needs_fix on the stored values,
 // FX_S x 256 columns at a time with all of their loads in flight, and the
 // marked ones listed in LDS.  Many marked (a row with an Inf or NaN): each
-// thread computes its own.  Few: each wave computes one output at a time,
-// its 64 lanes loading 64 products per step, FX_U steps at a time, which
-// the wave adds in ascending t (constant lane indices for full steps).
-// Blocks stride over the rows, so every block reaches the end.
+// thread computes its own.  Few: a wave per output, or the block where there
+// is one, loads FX_U products per thread and step, the next step's in flight,
+// and a wave adds them in ascending t from LDS, four to a read that all its
+// lanes share.  Random data mark a handful of outputs of 8192^2, so this is
+// bound by what one takes, a column of B with a cache line per element and T
+// dependent adds: 92 us (135 where one wave loads, 164 where it also fetches
+// its lanes' products one by one).  Blocks stride over the rows, so every
+// block reaches the end.
 constexpr int FX_S = 16, FX_U = 16;
 __global__ __launch_bounds__(256) void mm_fixup(const float *a, const float *b, float *c, MmPlan p,
                                                 const float *__restrict__ sA, const float *__restrict__ sB,
@@ -468,6 +474,7 @@ __global__ __launch_bounds__(256) void mm_fixup(const float *a, const float *b, 
                                                 const int *__restrict__ rowflag) {
   __shared__ int list[256 * FX_S];
   __shared__ int nlist;
+  __shared__ __align__(16) float prod[256 * FX_U];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   for (int64_t h = blockIdx.x; h < p.H; h += gridDim.x) {
     if (!rowflag[h]) continue;
@@ -504,34 +511,57 @@ __global__ __launch_bounds__(256) void mm_fixup(const float *a, const float *b, 
           crow[col * p.c_w] = pdl_dot_f32(arow, p.a_t, b + p.off[1] + col * p.b_w, p.b_t, p.T);
         }
       } else {
-        for (int i = w; i < n; i += 4) {
+        // G threads compute one output
+        auto dot = [&](auto group, int i) {
+          constexpr int G = decltype(group)::value, STEP = G * FX_U;
+          const int id = G == 64 ? lane : tid;
+          float *pr = prod + (G == 64 ? w * STEP : 0);
+          auto meet = [&]() {
+            if constexpr (G == 64) {   // LDS takes a wave's accesses in order
+              __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+              __builtin_amdgcn_wave_barrier();
+            } else {
+              __syncthreads();
+            }
+          };
           const int64_t col = w0 + list[i];
           const float *bcol = b + p.off[1] + col * p.b_w;
-          auto prod_at = [&](int64_t t0) {
-            const int64_t t = t0 + lane;
-            return t < p.T ? arow[t * p.a_t] * bcol[t * p.b_t] : 0.0f;
+          float v[FX_U];
+          auto load = [&](int64_t t0) {
+#pragma unroll
+            for (int u = 0; u < FX_U; u++) {
+              const int64_t t = t0 + G * u + id;
+              v[u] = t < p.T ? arow[t * p.a_t] * bcol[t * p.b_t] : 0.0f;
+            }
           };
           float cc = 0.0f;
-          for (int64_t t0 = 0; t0 < p.T; t0 += 64 * FX_U) {
-            float v[FX_U];
+          load(0);
+          for (int64_t t0 = 0; t0 < p.T; t0 += STEP) {
 #pragma unroll
-            for (int u = 0; u < FX_U; u++) v[u] = prod_at(t0 + 64 * u);
-            if (t0 + 64 * FX_U <= p.T) {
+            for (int u = 0; u < FX_U; u++) pr[G * u + id] = v[u];
+            meet();
+            if (t0 + STEP < p.T) load(t0 + STEP);
+            if (G == 64 || w == 0) {
+              const int m = p.T - t0 < STEP ? (int)(p.T - t0) : STEP;
+              int q = 0;
+              for (; q + 32 <= m; q += 32) {
+                Vec<float, 4> x[8];
 #pragma unroll
-              for (int u = 0; u < FX_U; u++)
+                for (int k = 0; k < 8; k++) x[k] = *reinterpret_cast<const Vec<float, 4> *>(&pr[q + 4 * k]);
 #pragma unroll
-                for (int l = 0; l < 64; l++) cc = cc + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[u]), l));
-            } else {
+                for (int k = 0; k < 8; k++)
 #pragma unroll
-              for (int u = 0; u < FX_U; u++) {
-                const int64_t tb = t0 + 64 * u;
-                const int m = p.T - tb < 64 ? (p.T - tb > 0 ? (int)(p.T - tb) : 0) : 64;
-                for (int l = 0; l < m; l++) cc = cc + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v[u]), l));
+                  for (int l = 0; l < 4; l++) cc = cc + x[k].v[l];
               }
+              for (; q < m; q++) cc = cc + pr[q];
             }
+            meet();
           }
-          if (lane == 0) crow[col * p.c_w] = cc;
-        }
+          if (id == 0) crow[col * p.c_w] = cc;
+        };
+        if (n == 1) dot(std::integral_constant<int, 256>(), 0);
+        else
+          for (int i = w; i < n; i += 4) dot(std::integral_constant<int, 64>(), i);
       }
       __syncthreads();   // the list is refilled for the next columns
     }
