@@ -260,8 +260,8 @@ pdlhip_error pdlhip_op_info(const char *op, int *npdls, int *nparents);
 /* A list of n independent matmults, item i = matmult(a[i], b[i], c[i]) with
  * the semantics of pdlhip_run_matmult (null c[i] are created).  No
  * reference counterpart: PDL runs such a list as a Perl loop of matmult
- * calls.  mode PDLHIP_LIST_QUEUE: one persistent launch fed by a device work
- * queue of (product, tile) items, largest inner dimension first, tile shape
+ * calls.  mode PDLHIP_LIST_QUEUE: one persistent launch over a device list of
+ * (product, tile) items, largest inner dimension first, kernel and tile shape
  * picked per shape class by a timing autotuner and cached; PDLHIP_LIST_EACH:
  * one launch per product (the comparison point).  Items that need a type
  * conversion or bad-value handling run through pdlhip_run_matmult. */
@@ -271,7 +271,7 @@ pdlhip_error pdlhip_run_matmult_list(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlh
 /* A prepared matmult list (no reference counterpart): the entries are
  * planned once as pdlhip_run_matmult_list plans them (outputs created),
  * their items and tile decompositions kept in HBM; each launch then runs
- * the whole list (PDLHIP_LIST_QUEUE: one persistent work-queue launch,
+ * the whole list (PDLHIP_LIST_QUEUE: one persistent launch,
  * PDLHIP_LIST_EACH: one launch per product) and allocates nothing, so it can
  * be captured in a HIP graph.  Entries with bad values, needing a type
  * conversion or of another type than the first are refused. */
@@ -348,10 +348,11 @@ pdlhip_error pdlhip_graph_destroy(void *graph);
 
 /* How float and double matmult compute (no reference counterpart: the
  * reference has a single scalar loop, Primitive.pd:211-245):
- *   SPLIT16   default; float: FP16 hi/lo split, 3 MFMA products, FP32
- *             accumulate (single products from 64 per side; broadcast batches
- *             of products with 16..64 per side; other shapes as FP32);
- *             double: FP64 MFMA from 8 per side
+ *   SPLIT16   default; double: FP64 MFMA from 8 per side; float: FP32 MFMA
+ *             from 8 per side, sums in parts of a few k, up to 8e9 operations
+ *             (up to 3e10 as the tuner picks); beyond that, and for broadcast
+ *             batches of products with 33..64 per side, FP16 hi/lo split, 3
+ *             MFMA products, FP32 accumulate; smaller sides as FP32
  *   FP32      plain SIMT kernel with fused multiply-add (float and double)
  *   PDLORDER  SIMT, multiply then add in ascending t: bit-identical to the
  *             reference's loop
