@@ -1139,12 +1139,12 @@ def _run(op, pdls, swap=0, m_size=None, dpar=None):
             _written(buf)
 
 
-class _Args(threading.local):
-    """One thread's argument block of pdlhip_run: the ndarrays' structs side by
-    side, the table of their addresses and the OtherPars.  It holds the
+class _Args:
+    """The argument block of one call of pdlhip_run: the ndarrays' structs side
+    by side, the table of their addresses and the OtherPars.  It holds the
     arguments of the call under way and nothing after it.  Building structs
     and pointers anew took most of an eager op's time: c = a*b + a and
-    sumover(c) over 48 x 50 doubles took 34.7 us, with the block 27.3."""
+    sumover(c) over 48 x 50 doubles took 34.7 us, with a kept block 27.3."""
     MAX = 6
 
     def __init__(self):
@@ -1167,7 +1167,14 @@ class _Args(threading.local):
         return self.run
 
 
-_args = _Args()
+class _Spare(threading.local):
+    """A thread's argument block while no call has it.  A call takes it out
+    and puts it back: Python may run other code of the same thread in the
+    middle of one (a signal handler, a finalizer the garbage collector calls),
+    and an op in there finds no block and makes its own."""
+
+
+_spare = _Spare()
 
 
 def _pdl_struct(nd):
@@ -1185,8 +1192,16 @@ _STATE_AT, _DIMS_AT, _INCS_AT, _DATA_AT = (L.Pdl.state.offset, L.Pdl.dims.offset
 
 def _call(op, pdls, swap=0, m_size=None, dpar=None):
     """the bare C ABI call (no dataflow bookkeeping)"""
+    A = _spare.__dict__.pop("args", None) or _Args()
+    try:
+        return _call_in(A, op, pdls, swap, m_size, dpar)
+    finally:
+        _spare.args = A
+
+
+def _call_in(A, op, pdls, swap, m_size, dpar):
+    """_call in the argument block A, which nothing else uses meanwhile"""
     n = len(pdls)
-    A = _args
     if n > A.MAX:
         raise PDLError(L.EUSERERROR, "pdlhip: %s: %d ndarrays" % (op, n))
     mem, table_at, o = A.mem, A.table_at, 0
