@@ -20,10 +20,10 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 # No FMA contraction (PDL's a*b+a rounds twice), wrapping signed ints (PDL
-# is built with -fwrapv), no packed-FP32 instructions.
+# is built with -fwrapv), no packed-FP32 instructions, no status dropped.
 FLAGS = ["--offload-arch=" + ARCH, "-O3", "-fPIC", "-std=c++17", "-ffp-contract=off", "-fwrapv",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-         "-Wno-unused-command-line-argument", "-I" + CSRC]
+         "-Wno-unused-command-line-argument", "-Werror=unused-value", "-I" + CSRC]
 
 NTYPES = 11
 

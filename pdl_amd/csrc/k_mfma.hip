@@ -883,15 +883,17 @@ hipError_t launch_mfma_f32(const MmPlan &p, const float *a, const float *b, floa
   if (e == hipSuccess) e = prep_operand(b, o[1], p.b_w, p.b_t, p.W, p.T, Wp, Kp, sB, dB, nullptr, Bh, B8, fp8, s);
   const int64_t ntm = Hp / BMr, ntn = Wp / BNr;
   if (e == hipSuccess) {
-    if (fp8 && big)
-      hipLaunchKernelGGL((fp8_gemm_big<256, 256, 4, 2>), dim3((unsigned)(ntm * ntn)), dim3(512), 0, s, A8, B8, sA, sB,
-                         dA, dB, rowflag, c, p, Kp, ntm, ntn);
-    else if (fp8)
-      hipLaunchKernelGGL(fp8_gemm, dim3((unsigned)(ntm * ntn)), dim3(256), 0, s, A8, B8, sA, sB, dA, dB, rowflag, c,
-                         p, Kp, ntm, ntn);
-    else
-      launch_split16(big, Ah, Bh, sA, sB, dA, dB, rowflag, c, p, Kp, ntm, ntn, s);
-    e = hipGetLastError();
+    if (!fp8) {
+      e = launch_split16(big, Ah, Bh, sA, sB, dA, dB, rowflag, c, p, Kp, ntm, ntn, s);
+    } else {
+      if (big)
+        hipLaunchKernelGGL((fp8_gemm_big<256, 256, 4, 2>), dim3((unsigned)(ntm * ntn)), dim3(512), 0, s, A8, B8, sA,
+                           sB, dA, dB, rowflag, c, p, Kp, ntm, ntn);
+      else
+        hipLaunchKernelGGL(fp8_gemm, dim3((unsigned)(ntm * ntn)), dim3(256), 0, s, A8, B8, sA, sB, dA, dB, rowflag, c,
+                           p, Kp, ntm, ntn);
+      e = hipGetLastError();
+    }
   }
   if (e == hipSuccess) {
     const int64_t fb = p.H < 2048 ? p.H : 2048;
