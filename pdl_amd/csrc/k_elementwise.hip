@@ -341,7 +341,7 @@ static hipError_t binop_T_OP(const EwPlan &p, const void *va, const void *vb, vo
             if (!unit && p.inc[k][d] % V4) vec = false;
           }
         }
-        if (nblk < (int64_t)1 << 31) {
+        if (nblk < GRID_BLOCKS) {
           const bool stream = streaming_read((size_t)p.n * sizeof(T) * 2);
 #define TILE_LAUNCH(TM, VV) hipLaunchKernelGGL((ew_tile<T, OP, TM, VV>), dim3((unsigned)nblk), dim3(EW_THREADS), 0, s, \
                                                a, b, c, p, q, nti, ntj, stream)
@@ -361,7 +361,7 @@ static hipError_t binop_T_OP(const EwPlan &p, const void *va, const void *vb, vo
     int64_t chunk = p.dims[0] < 8192 ? p.dims[0] : 8192;
     int64_t cpr = (p.dims[0] + chunk - 1) / chunk;
     int64_t nblk = rows * cpr;
-    if (nblk < (int64_t)1 << 31) {
+    if (nblk < GRID_BLOCKS) {
       if (bad)
         hipLaunchKernelGGL((ew_rows<T, OP, true>), dim3((unsigned)nblk), dim3(EW_THREADS), 0, s, a, b, c, p, cpr,
                            chunk, bi[0], bi[1], cbad);

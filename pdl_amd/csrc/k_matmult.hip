@@ -73,11 +73,12 @@ __global__ __launch_bounds__(256) void mm_simt(const T *__restrict__ a, const T 
                                                MmPlan p, int64_t ntm, int64_t ntn, int a_tfast, int b_wfast) {
   __shared__ T As[SB_K][SB_M + 1];
   __shared__ T Bs[SB_K][SB_N + 1];
-  int64_t blk = blockIdx.x;
+  int64_t blk = grid_block();
   const int64_t tm = blk % ntm;
   blk /= ntm;
   const int64_t tn = blk % ntn;
   const int64_t bidx = blk / ntn;
+  if (bidx >= p.nbatch) return;
   int64_t o[3];
   mm_batch_offsets(p, bidx, o);
   const int tid = threadIdx.x;
@@ -178,14 +179,15 @@ static hipError_t matmult_T(const MmPlan &p, const void *va, const void *vb, voi
   const int64_t ntm = (p.H + SB_M - 1) / SB_M, ntn = (p.W + SB_N - 1) / SB_N;
   const int64_t blocks = ntm * ntn * p.nbatch;
   if (blocks >= ((int64_t)1 << 31)) return hipErrorInvalidConfiguration;
+  const dim3 grid = grid_of(blocks);
   const int a_tfast = (p.a_t == 1 || p.a_h != 1) ? 1 : 0;
   const int b_wfast = (p.b_w == 1 || p.b_t != 1) ? 1 : 0;
   const bool fused = IsFloat<T>::v && mode != PDLHIP_MM_PDLORDER;
   if (fused)
-    hipLaunchKernelGGL((mm_simt<T, true>), dim3((unsigned)blocks), dim3(256), 0, s, a, b, c, p, ntm, ntn, a_tfast,
+    hipLaunchKernelGGL((mm_simt<T, true>), grid, dim3(256), 0, s, a, b, c, p, ntm, ntn, a_tfast,
                        b_wfast);
   else
-    hipLaunchKernelGGL((mm_simt<T, false>), dim3((unsigned)blocks), dim3(256), 0, s, a, b, c, p, ntm, ntn, a_tfast,
+    hipLaunchKernelGGL((mm_simt<T, false>), grid, dim3(256), 0, s, a, b, c, p, ntm, ntn, a_tfast,
                        b_wfast);
   return hipGetLastError();
 }

@@ -613,7 +613,7 @@ static hipError_t prep_operand(const float *src, int64_t o, int64_t inc_r, int64
 }
 
 // Small float products (33..64 per side), typically broadcast batches:
-// a block of 4 waves per product (a grid capped at 2^31 - 1 blocks loops,
+// a block of 4 waves per product (a grid capped at 2^24 - 1 blocks loops,
 // fetching its next product's operands while it multiplies the current
 // one; a persistent grid of resident blocks measured slower), nothing
 // staged outside the kernel.  A
@@ -840,8 +840,8 @@ hipError_t launch_mfma_f32(const MmPlan &p, const float *a, const float *b, floa
   // small products (broadcast batches of them in one launch)
   if (!fp8 && small_split16(p)) {
     // a block per product (the block loop then runs once); more products
-    // than 2^31 - 1 loop
-    const int64_t blocks = p.nbatch < ((int64_t)1 << 31) - 1 ? p.nbatch : ((int64_t)1 << 31) - 1;
+    // than a grid holds blocks loop
+    const int64_t blocks = p.nbatch < GRID_BLOCKS ? p.nbatch : GRID_BLOCKS - 1;
     // 64x64x64 products with unit-stride k (A) and w (B), every product's
     // rows 16-byte aligned: 16-byte staging loads
     bool vec = p.H == SMM && p.W == SMM && p.T == SMM && p.a_t == 1 && p.b_w == 1 && p.a_h % 4 == 0 &&

@@ -441,8 +441,8 @@ __global__ __launch_bounds__(RT) void scan_seq(const Tin *__restrict__ a, RedPla
   auto out = [&](int64_t k) { return (Tout *)(sq_lds + 16 * G) + (int)(k & 1) * G * po; };
   auto in = [&](int64_t k) { return (Tin *)(sq_lds + 16 * G + 2 * G * po * sizeof(Tout)) + (int)(k & 1) * G * pi; };
   const int tid = threadIdx.x, lc = __builtin_ctz(C), lg = __builtin_ctz(G);
-  const int64_t e0 = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * G;
-  if (e0 >= p.nout) return;   // (the grid's last row of blocks)
+  const int64_t e0 = grid_block() * G;
+  if (e0 >= p.nout) return;
   const int rows = p.nout - e0 < G ? (int)(p.nout - e0) : G;
   if (tid < rows) {
     int64_t off[MAXP];
@@ -607,10 +607,9 @@ static hipError_t seq_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
   auto nfast = [&](int q) { return p.nout == 1 || p.nd == 0 || mag(p.inc_n[q]) <= mag(p.inc[q][0]); };
   const size_t lds = 16 * (size_t)G + 2 * (size_t)G * (sizeof(Tin) * sq_pitch<Tin, Tout>(C, one) +
                                                        sizeof(Tout) * sq_pitch<Tout, Tout>(C, one));
-  // a dimension of a grid holds fewer than 2^32 threads: 2^24 blocks
-  const int64_t blocks = (p.nout + G - 1) / G, ny = (blocks + (1 << 22) - 1) >> 22;
-  if (ny > 65535) return hipErrorInvalidConfiguration;
-  const dim3 grid((unsigned)((blocks + ny - 1) / ny), (unsigned)ny);
+  const int64_t blocks = (p.nout + G - 1) / G;
+  if (blocks >= ((int64_t)1 << 31)) return hipErrorInvalidConfiguration;
+  const dim3 grid = grid_of(blocks);
   if (one)
     hipLaunchKernelGGL((scan_seq<OP, Tin, Tout, BAD, true>), grid, dim3(RT), lds, s, a, p, o, ba, G, C,
                        nfast(0) ? 1 : 0, nfast(1) ? 1 : 0);

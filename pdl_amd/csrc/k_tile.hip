@@ -36,6 +36,7 @@ template <class T> struct TilePlan {
   MmPlan p;
   int64_t ntm, ntn;    // tiles of one product
   int64_t nwhole;      // tiles summed over all of t; the others in S parts of kc
+  int64_t nblocks;
   int32_t S;
   int64_t kc;
   T *part;
@@ -69,7 +70,8 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && !FINE ? 3 : 4) void tile_gem
   const MmPlan &p = g.p;
   // whole tiles first, each XCD (block b runs on XCD b % 8) a contiguous
   // share of them, then the parts
-  int64_t t = blockIdx.x, kb = 0, ke = p.T;
+  int64_t t = grid_block(), kb = 0, ke = p.T;
+  if (t >= g.nblocks) return;
   int part = -1;
   if (t < g.nwhole) {
     if (g.nwhole % 8 == 0) t = (t % 8) * (g.nwhole / 8) + t / 8;
@@ -138,7 +140,8 @@ static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hip
   g.nwhole = g.S > 1 ? nt - rest : nt;
   if (g.S == 1) g.kc = p.T;
   const bool ak = p.a_t == 1, bk = p.b_t == 1;
-  const dim3 grid((unsigned)(g.nwhole + (nt - g.nwhole) * g.S));
+  g.nblocks = g.nwhole + (nt - g.nwhole) * g.S;
+  const dim3 grid = grid_of(g.nblocks);
   // (float) sums of 8 k rather than 32 where all of t is three stages or less
   auto go = [&](auto fine) {
     constexpr bool F = decltype(fine)::value;
