@@ -335,8 +335,12 @@ pdlhip_error pdlhip_ragged_free(pdlhip_ragged *handle);
  * library's cache (no hipMalloc, no synchronisation): an op whose scratch
  * (float matmult packing, long-row reduction partials, converted copies,
  * created outputs) is not cached fails with PDLHIP_EUSERERROR, so run each
- * op once before capturing it.  Blocks an op releases during the capture
- * stay reserved for the graph until pdlhip_graph_destroy.  Calls that wait
+ * op once before capturing it.  Three kinds of op need no earlier run: the
+ * partial results of strided reductions, of products cut along t and of long
+ * integer scans are allocated (hipMalloc, with the thread's capture mode
+ * relaxed) where none are cached; the ops of one graph share them.  Blocks
+ * an op releases during the capture stay reserved for the graph until
+ * pdlhip_graph_destroy.  Calls that wait
  * for the stream (upload, download, synchronize, ragged bad flags,
  * minimum_n_ind/maximum_n_ind with bad values, list and ragged prepare) are
  * refused during a capture.  The handle from pdlhip_graph_end is the

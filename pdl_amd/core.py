@@ -1444,8 +1444,9 @@ def tune_stats():
 class Graph:
     """A HIP graph of the work `fn` enqueues on the library's stream.  Ops
     may take scratch memory only from the library's cache while capturing
-    (run an op once before capturing it); blocks they release stay with the
-    graph until destroy().  Ops that wait for the stream (downloads, bad-value
+    (run an op once before capturing it; the partial results of strided
+    reductions, cut products and long integer scans are allocated where none
+    are cached); blocks they release stay with the graph until destroy().  Ops that wait for the stream (downloads, bad-value
     *_n_ind, ragged bad flags) are refused."""
 
     def __init__(self, fn):

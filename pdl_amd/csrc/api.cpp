@@ -116,6 +116,7 @@ struct Global {
   // them is destroyed
   bool capturing = false;
   std::vector<void *> pinned;
+  std::multimap<size_t, void *> spare;   // partials_free'd in the capture under way
   void *noalloc_scratch = nullptr;   // device address of `scratch`
   // PDL's random-number stream (one state: PDL with autopthread off)
   uint64_t rng[4] = {0, 0, 0, 0};
@@ -176,7 +177,7 @@ static void release_cached() {
   g_cache.cached = 0;
 }
 
-void *dev_alloc(size_t n) {
+static void *dev_alloc(size_t n, bool while_capturing) {
   if (g_noalloc) return nullptr;
   size_t sz = round_size(n);
   std::lock_guard<std::mutex> lk(g_cache.mu);
@@ -187,9 +188,17 @@ void *dev_alloc(size_t n) {
     g_cache.freelist.erase(it);
     return p;
   }
-  if (capturing()) return nullptr;   // no hipMalloc or synchronisation inside a capture
   void *p = nullptr;
-  if (hipMalloc(&p, sz) != hipSuccess) {
+  if (capturing()) {
+    if (!while_capturing) return nullptr;   // no hipMalloc or synchronisation inside a capture
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // (other modes forbid hipMalloc)
+    hipError_t e = hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) {
+      e = hipMalloc(&p, sz);
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    if (e != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+  } else if (hipMalloc(&p, sz) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipStreamSynchronize(g.stream);
     release_cached();
@@ -199,6 +208,8 @@ void *dev_alloc(size_t n) {
   g_cache.owned[p] = sz;
   return p;
 }
+
+void *dev_alloc(size_t n) { return dev_alloc(n, false); }
 
 bool dev_free(void *p) {
   if (!p) return true;
@@ -222,6 +233,36 @@ bool dev_free(void *p) {
 
 void *scratch_alloc(size_t bytes) { return dev_alloc(bytes); }
 void scratch_free(void *p) { dev_free(p); }
+
+// Partial results between the two kernels of an op that could also do without
+// them, in another order of summation and many times slower (strided
+// reductions, products and integer scans cut into parts).  During a capture
+// they are allocated where none are cached, so that a graph's results and
+// speed are the eager call's whatever ran before it.  The kernels of one
+// graph run in order and share what is released on the way; null when memory
+// is short.
+void *partials_alloc(size_t bytes) {
+  {
+    std::lock_guard<std::mutex> lk(g_cache.mu);
+    const size_t sz = round_size(bytes);
+    auto it = g.spare.lower_bound(sz);
+    if (it != g.spare.end() && it->first <= sz + sz / 4) {
+      void *p = it->second;
+      g.spare.erase(it);
+      return p;
+    }
+  }
+  return dev_alloc(bytes, true);
+}
+
+void partials_free(void *p) {
+  if (!g.capturing) {
+    dev_free(p);
+    return;
+  }
+  std::lock_guard<std::mutex> lk(g_cache.mu);
+  g.spare.insert({g_cache.owned[p], p});
+}
 
 // ------------------------------------------------------------------ signatures
 enum Family { FAM_BIOP, FAM_BIFUNC, FAM_ASSGN, FAM_RED, FAM_NIND, FAM_MM, FAM_UFUNC, FAM_BADOP, FAM_INDEX };
@@ -2741,6 +2782,8 @@ pdlhip_error pdlhip_graph_end(void **graph) {
   {
     std::lock_guard<std::mutex> lk(g_cache.mu);
     pinned.swap(g.pinned);
+    for (auto &kv : g.spare) pinned.push_back(kv.second);
+    g.spare.clear();
   }
   if (e != hipSuccess) {
     unpin(pinned);

@@ -39,6 +39,8 @@ namespace pdlhip {
 
 void *scratch_alloc(size_t bytes);
 void scratch_free(void *p);
+void *partials_alloc(size_t bytes);
+void partials_free(void *p);
 
 __device__ inline void out_offsets(const RedPlan &p, int64_t e, int64_t *off) {
   for (int k = 0; k < p.npdl; k++) off[k] = p.off[k];
@@ -676,9 +678,8 @@ __global__ __launch_bounds__(RT) void red_thread(const Tin *__restrict__ a, RedP
 // launches red_grid: lanes along n where its stride is the smaller of the
 // two, a wave's worth of outputs side by side otherwise; n is cut into chunks
 // of at least 32 elements per thread until there are about 1024 blocks (four
-// per CU; 2048 measured 22.5 + 7.0 us for that table).  Without scratch for
-// the partials (a capture with none cached, the allocation-free entry's
-// limit) n stays whole and every call still runs.
+// per CU; 2048 measured 22.5 + 7.0 us for that table).  Where memory for the
+// partials cannot be had, n stays whole and the call still runs.
 template <int OP, class Tin, class Tout, class Tacc, bool BAD>
 static hipError_t grid_launch(const RedPlan &p, const Tin *a, const Outs &o, const BadInfo &ba, hipStream_t s) {
   const int64_t in0 = p.inc_n[0] < 0 ? -p.inc_n[0] : p.inc_n[0];
@@ -711,7 +712,7 @@ static hipError_t grid_launch(const RedPlan &p, const Tin *a, const Outs &o, con
   }
   Part<Tin, Tacc> *parts = nullptr;
   if (nchunk > 1) {
-    parts = (Part<Tin, Tacc> *)(p.scratch ? p.scratch : scratch_alloc(sizeof(*parts) * (size_t)p.nout * (size_t)nchunk));
+    parts = (Part<Tin, Tacc> *)(p.scratch ? p.scratch : partials_alloc(sizeof(*parts) * (size_t)p.nout * (size_t)nchunk));
     if (!parts) nchunk = 1;
   } else {
     nchunk = 1;
@@ -727,7 +728,7 @@ static hipError_t grid_launch(const RedPlan &p, const Tin *a, const Outs &o, con
                        ba, LE, R, nchunk, clen, parts);
   if (parts) split2_launch<OP, Tin, Tout, Tacc, BAD>(p, nchunk, parts, o, s);
   const hipError_t err = hipGetLastError();
-  if (parts && !p.scratch) scratch_free(parts);
+  if (parts && !p.scratch) partials_free(parts);
   return err;
 }
 
@@ -797,8 +798,8 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
           clen = (p.n + want - 1) / want;
           clen = clen < 8192 ? 8192 : (clen + SC_CH - 1) / SC_CH * SC_CH;
           nchunk = (p.n + clen - 1) / clen;
-          totals = (Tout *)scratch_alloc(sizeof(Tout) * (size_t)(p.nout * nchunk));
-          if (!totals) { nchunk = 1; clen = p.n; }   // none cached during a capture: a block per row
+          totals = (Tout *)partials_alloc(sizeof(Tout) * (size_t)(p.nout * nchunk));
+          if (!totals) { nchunk = 1; clen = p.n; }   // out of memory: a block per row
         }
         if (totals)
           hipLaunchKernelGGL((scan_totals<OP, Tin, Tout, BAD>), dim3((unsigned)(p.nout * nchunk)), dim3(RT), 0, s, a, p,
@@ -807,7 +808,7 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
         hipLaunchKernelGGL((scan_rows<OP, Tin, Tout, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba, nchunk,
                            clen, totals);
         const hipError_t err = hipGetLastError();
-        if (totals) scratch_free(totals);
+        if (totals) partials_free(totals);
         return err;
       }
     }

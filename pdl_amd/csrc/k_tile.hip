@@ -29,8 +29,8 @@
 
 namespace pdlhip {
 
-void *scratch_alloc(size_t bytes);
-void scratch_free(void *p);
+void *partials_alloc(size_t bytes);
+void partials_free(void *p);
 
 template <class T> struct TilePlan {
   MmPlan p;
@@ -134,8 +134,8 @@ static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hip
   if (g.S > 1) {
     g.kc = ((p.T + g.S - 1) / g.S + TILE_K<T> - 1) / TILE_K<T> * TILE_K<T>;
     g.S = (int)((p.T + g.kc - 1) / g.kc);
-    g.part = (T *)scratch_alloc(sizeof(T) * (size_t)(rest * g.S * BM * BN));
-    if (!g.part) g.S = 1;   // none cached during a capture: whole tiles
+    g.part = (T *)partials_alloc(sizeof(T) * (size_t)(rest * g.S * BM * BN));
+    if (!g.part) g.S = 1;   // out of memory: whole tiles
   }
   g.nwhole = g.S > 1 ? nt - rest : nt;
   if (g.S == 1) g.kc = p.T;
@@ -159,7 +159,7 @@ static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hip
   if (g.part)
     hipLaunchKernelGGL((tile_join<T, BM, BN>), dim3((unsigned)((nt - g.nwhole) * (BM * BN / 256))), dim3(256), 0, s, c, g);
   const hipError_t e = hipGetLastError();
-  if (g.part) scratch_free(g.part);
+  if (g.part) partials_free(g.part);
   return e;
 }
 
