@@ -241,9 +241,10 @@ pdlhip_error pdlhip_writeback_rangeb(pdlhip_pdl *parent, pdlhip_pdl *ind, const 
  * cannot allocate device memory (code under HIP graph capture, tight
  * serving loops).  It allocates nothing: the output must exist and the
  * input and output must already have the types the op computes in (no
- * converted copy), else PDLHIP_EUSERERROR.  The long-row split keeps its
- * per-chunk partials in a 256 KiB array the library reserves on each GPU
- * (any input size fits; a launch that needed more would be refused).  All
+ * converted copy), else PDLHIP_EUSERERROR.  Long rows and strided ones keep
+ * the partials of their chunks in a 7 MiB array the library reserves on each
+ * GPU (any input size fits; a launch that needed more would be refused); the
+ * results have the bits of pdlhip_run.  All
  * calls on one GPU share that array: calls that overlap on one GPU (other
  * streams, graphs replayed concurrently) race. */
 pdlhip_error pdlhip_run_reduce_noalloc(const char *op, pdlhip_pdl *a, pdlhip_pdl *b);

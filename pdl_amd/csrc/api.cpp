@@ -42,12 +42,14 @@ namespace pdlhip {
 static thread_local std::string g_msg;
 
 // ------------------------------------------------------------------ allocation-free reductions
-// The scratch of pdlhip_run_reduce_noalloc: the long-row reductions'
-// per-chunk partials (at most 2048 + 1023 of them, under 200 KiB) live in
-// this array instead of a cached hipMalloc block.  Each GPU holds its own
+// The scratch of pdlhip_run_reduce_noalloc: the partials of long rows (at
+// most 2048 + 511 of them) and of strided ones (fewer than 2048 blocks of 64
+// outputs, 56 bytes each: under 7 MiB) live in this array instead of a cached
+// hipMalloc block.  It holds every launch's, so the rows are cut as in
+// pdlhip_run and both entries give the same bits.  Each GPU holds its own
 // copy until the process ends; host code uses the device address from
 // hipGetSymbolAddress (pdlhip_init), never the array's name.
-constexpr size_t NOALLOC_BYTES = (size_t)256 << 10;
+constexpr size_t NOALLOC_BYTES = (size_t)7 << 20;
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 static thread_local bool g_noalloc = false;   // inside pdlhip_run_reduce_noalloc
 static thread_local bool g_writeback = false; // inside pdlhip_writebackdata: run the op's BackCode

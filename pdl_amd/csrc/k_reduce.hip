@@ -706,13 +706,12 @@ static hipError_t grid_launch(const RedPlan &p, const Tin *a, const Outs &o, con
   int64_t nchunk = (1024 + ngroup - 1) / ngroup;
   const int64_t most = p.n / ((int64_t)R * 32);
   nchunk = nchunk < most ? nchunk : most;
-  if (p.scratch) {
-    const int64_t fit = p.scratch_bytes / (int64_t)(sizeof(Part<Tin, Tacc>) * (size_t)p.nout);
-    nchunk = nchunk < fit ? nchunk : fit;
-  }
+  static_assert(sizeof(Part<Tin, Tacc>) <= 56, "the caller's scratch counts on it");
   Part<Tin, Tacc> *parts = nullptr;
   if (nchunk > 1) {
-    parts = (Part<Tin, Tacc> *)(p.scratch ? p.scratch : partials_alloc(sizeof(*parts) * (size_t)p.nout * (size_t)nchunk));
+    const size_t need = sizeof(*parts) * (size_t)p.nout * (size_t)nchunk;
+    if (p.scratch && need > (size_t)p.scratch_bytes) return hipErrorOutOfMemory;
+    parts = (Part<Tin, Tacc> *)(p.scratch ? p.scratch : partials_alloc(need));
     if (!parts) nchunk = 1;
   } else {
     nchunk = 1;
