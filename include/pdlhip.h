@@ -353,11 +353,12 @@ pdlhip_error pdlhip_graph_destroy(void *graph);
 
 /* How float and double matmult compute (no reference counterpart: the
  * reference has a single scalar loop, Primitive.pd:211-245):
- *   SPLIT16   default; double: FP64 MFMA from 8 per side; float: FP32 MFMA
- *             from 8 per side, sums in parts of a few k, up to 8e9 operations
- *             (up to 3e10 as the tuner picks); beyond that, and for broadcast
- *             batches of products with 33..64 per side, FP16 hi/lo split, 3
- *             MFMA products, FP32 accumulate; smaller sides as FP32
+ *   SPLIT16   default; double: FP64 MFMA from 8 per side; float: by its
+ *             sizes alone, either FP32 MFMA with sums in parts of a few k
+ *             (from 8 per side), or an FP16 hi/lo split, 3 MFMA products,
+ *             FP32 accumulate: beyond 3e10 operations, below that where it is
+ *             the faster one (from about 7e9), and for products with 33..64
+ *             per side; smaller sides as FP32
  *   FP32      plain SIMT kernel with fused multiply-add (float and double)
  *   PDLORDER  SIMT, multiply then add in ascending t: bit-identical to the
  *             reference's loop
@@ -392,6 +393,8 @@ pdlhip_error pdlhip_readdata(const char *op, int datatype, int bvalflag,
  * GEMM block shapes) are timed once per shape class and kept in
  * $PDLHIP_TUNE_FILE (default
  * ~/.cache/pdlhip/tune-<arch>.txt); PDLHIP_TUNE=0 keeps the default rules.
+ * The block shapes of a product all give the same bits; the kernels of a list
+ * differ within the bounds of its precision mode.
  * The counts of choices this process measured and reused from the file. */
 pdlhip_error pdlhip_tune_stats(int64_t *measured, int64_t *reused);
 

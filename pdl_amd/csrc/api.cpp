@@ -38,6 +38,9 @@
 
 namespace pdlhip {
 
+bool tile_takes_f32(const MmPlan &p);                  // k_tile.hip
+std::vector<int> tile_widths_f32(const MmPlan &p);
+
 // ------------------------------------------------------------------ errors
 static thread_local std::string g_msg;
 
@@ -1166,19 +1169,18 @@ static pdlhip_error readdata(const Sig &s, int T, bool bad, const Brc &b, pdlhip
       return ok();
     }
     if (g.defer) g.defer->missed++;
-    // the autotuner's engine for float products: the FP32 matrix cores (64),
-    // or FP16 split / FP8 blocks of 128x128 or 256x256, timed into a scratch
-    // output
+    // the autotuner's block shape for large float products, timed into a
+    // scratch output: 64x64 or 64x32 on the FP32 matrix cores, 128x128 or
+    // 256x256 for the FP16 split and FP8.  All shapes of an engine give the
+    // same bits; the engine goes by the sizes.
     const bool mm16 = T == PDLHIP_F && (g.mm_mode == PDLHIP_MM_SPLIT16 || g.mm_mode == PDLHIP_MM_FP8);
     if (!bad && p.nbatch == 1 && mm16 && p.H >= 512 && p.W >= 512 && p.T >= 32) {
       char fam[160];
+      const bool tiles = g.mm_mode == PDLHIP_MM_SPLIT16 && tile_takes_f32(p);
       snprintf(fam, sizeof fam, "matmult:%s:%s:h2^%d:w2^%d:t2^%d", type_name(T),
-               g.mm_mode == PDLHIP_MM_FP8 ? "fp8" : "tile_or_ring", ilog2(p.H), ilog2(p.W), ilog2(p.T));
-      std::vector<int> cands = {128, 256};
-      int dflt = (p.H >= 1024 && p.W >= 1024) ? 256 : 128;
-      const double flops = 2.0 * (double)p.H * (double)p.W * (double)p.T;
-      if (g.mm_mode == PDLHIP_MM_SPLIT16 && flops <= 3e10) cands.push_back(64);
-      if (g.mm_mode == PDLHIP_MM_SPLIT16 && flops <= 8e9) dflt = 64;
+               g.mm_mode == PDLHIP_MM_FP8 ? "fp8" : tiles ? "tile" : "ring", ilog2(p.H), ilog2(p.W), ilog2(p.T));
+      const std::vector<int> cands = tiles ? tile_widths_f32(p) : std::vector<int>{128, 256};
+      const int dflt = tiles ? 64 : (p.H >= 1024 && p.W >= 1024) ? 256 : 128;
       void *tc = nullptr;
       auto run_one = [&](int cand) -> hipError_t {
         if (!tc) tc = dev_alloc((size_t)p.H * p.W * type_size(T));
@@ -1190,7 +1192,7 @@ static pdlhip_error readdata(const Sig &s, int T, bool bad, const Brc &b, pdlhip
         q.c_h = p.W;
         return matmult_dispatch(T, q, pdls[0]->data, pdls[1]->data, tc, false, bi, g.mm_mode, st);
       };
-      p.variant = tune(fam, cands, dflt, run_one);
+      p.variant = cands.size() > 1 ? tune(fam, cands, dflt, run_one) : dflt;
       if (tc) dev_free(tc);
     }
     e = matmult_dispatch(T, p, pdls[0]->data, pdls[1]->data, pdls[2]->data, bad, bi, g.mm_mode, st);

@@ -21,9 +21,9 @@
 namespace pdlhip {
 
 hipError_t launch_mfma_f32(const MmPlan &p, const float *a, const float *b, float *c, int mode, hipStream_t s);
-bool small_split16(const MmPlan &p);   // whether launch_mfma_f32's small-product kernel takes it
 hipError_t launch_tile_f64(const MmPlan &p, const double *a, const double *b, double *c, hipStream_t s);
 hipError_t launch_tile_f32(const MmPlan &p, const float *a, const float *b, float *c, hipStream_t s);
+bool tile_takes_f32(const MmPlan &p);   // whether the default mode runs p on launch_tile_f32
 
 __device__ inline void mm_batch_offsets(const MmPlan &p, int64_t bidx, int64_t *o) {
   o[0] = p.off[0]; o[1] = p.off[1]; o[2] = p.off[2];
@@ -151,16 +151,7 @@ static hipError_t matmult_T(const MmPlan &p, const void *va, const void *vb, voi
     return hipGetLastError();
   }
   if constexpr (sizeof(T) == 4 && IsFloat<T>::v) {
-    // The default mode runs on the FP32 matrix cores up to MM_TILE_FLOPS,
-    // where the FP16 split's packing costs more than its faster product
-    // gains (1024^3: 36 against 70 us; 1500^3: 94 against 139; 2048^3: 192
-    // against 169), unless the autotuner measured otherwise (variant 64, 128
-    // or 256), and batches of products; 33..64 per side have a kernel of
-    // their own there.
-    constexpr double MM_TILE_FLOPS = 8e9;
-    const bool small = small_split16(p);
-    if (mode == PDLHIP_MM_SPLIT16 && !small &&
-        (p.variant ? p.variant == 64 : p.nbatch != 1 || 2.0 * (double)p.H * (double)p.W * (double)p.T <= MM_TILE_FLOPS)) {
+    if (mode == PDLHIP_MM_SPLIT16 && tile_takes_f32(p)) {
       hipError_t e = launch_tile_f32(p, (const float *)a, (const float *)b, (float *)c, s);
       if (e != hipErrorNotSupported) return e;
     }

@@ -835,6 +835,9 @@ bool small_split16(const MmPlan &p) {
          fits32(p.H, p.a_h, p.T, p.a_t) && fits32(p.W, p.b_w, p.T, p.b_t);
 }
 
+// one product, and where a 128x128 tile of it is mostly useful
+bool single_split16(const MmPlan &p) { return p.nbatch == 1 && p.H >= 64 && p.W >= 64 && p.T >= 32; }
+
 hipError_t launch_mfma_f32(const MmPlan &p, const float *a, const float *b, float *c, int mode, hipStream_t s) {
   const bool fp8 = (mode == PDLHIP_MM_FP8);
   // small products (broadcast batches of them in one launch)
@@ -851,9 +854,7 @@ hipError_t launch_mfma_f32(const MmPlan &p, const float *a, const float *b, floa
     else hipLaunchKernelGGL(split16_small<false>, dim3((unsigned)blocks), dim3(256), 0, s, a, b, c, p);
     return hipGetLastError();
   }
-  // otherwise one matrix product per call (broadcast batches use the SIMT
-  // kernel), and only where a 128x128 tile is mostly useful
-  if (p.nbatch != 1 || p.H < 64 || p.W < 64 || p.T < 32) return hipErrorNotSupported;
+  if (!single_split16(p)) return hipErrorNotSupported;
   // 256x256 blocks once both sides fill them (FP8 then steps k by 64), or as
   // the autotuner picked (variant 128 / 256)
   const bool big = p.variant ? p.variant == 256 : (p.H >= 1024 && p.W >= 1024);

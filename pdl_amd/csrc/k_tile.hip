@@ -22,6 +22,7 @@
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
+#include <vector>
 
 #include "device.hpp"
 #include "launch.hpp"
@@ -31,6 +32,8 @@ namespace pdlhip {
 
 void *partials_alloc(size_t bytes);
 void partials_free(void *p);
+bool small_split16(const MmPlan &p);    // k_mfma.hip: what the FP16 split's batch kernel takes
+bool single_split16(const MmPlan &p);   // and its large product
 
 template <class T> struct TilePlan {
   MmPlan p;
@@ -109,6 +112,22 @@ __global__ __launch_bounds__(256) void tile_join(T *__restrict__ c, TilePlan<T> 
     c[o[2] + (tn * BN + wv) * g.p.c_w + (tm * BM + h) * g.p.c_h] = s;
 }
 
+// Into how many parts the tiles past the last multiple of 256 (a tile per CU)
+// are cut: whole, they leave CUs idle for a whole tile's time.  S parts make
+// that ceil(rest * S / 256) / S of it, for a second launch and the parts'
+// traffic (about 4 us); a part keeps at least 64 k.
+template <class T> static int tile_parts(int64_t rest, int BM, int BN, int64_t K) {
+  constexpr double CU_FLOPS = sizeof(T) == 8 ? 0.24e6 : 0.44e6;   // per us and CU, as measured
+  const double tile_us = 2.0 * BM * BN * (double)K / CU_FLOPS;
+  int parts = 1;
+  double best = rest ? tile_us : 0.0;
+  for (int S = 2; S <= 16 && rest && K / S >= 64; S++) {
+    const double us = tile_us * (double)((rest * S + 255) / 256) / S + 4.0 + (double)(rest * S * BM * BN * 2 * sizeof(T)) / 3e6;
+    if (us < best) { best = us; parts = S; }
+  }
+  return parts;
+}
+
 template <class T, int BM, int BN, int WR, int WC>
 static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hipStream_t s) {
   TilePlan<T> g;
@@ -117,19 +136,8 @@ static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hip
   g.ntn = (p.W + BN - 1) / BN;
   const int64_t nt = g.ntm * g.ntn * p.nbatch;
   if (nt >= ((int64_t)1 << 30)) return hipErrorNotSupported;
-  // Tiles past the last multiple of 256 (a tile per CU) leave CUs idle for a
-  // whole tile's time.  Cutting each into S parts makes that ceil(rest * S /
-  // 256) / S of it, for a second launch and the parts' traffic (about 4 us);
-  // a part keeps at least 64 k.
-  constexpr double CU_FLOPS = sizeof(T) == 8 ? 0.24e6 : 0.44e6;   // per us and CU, as measured
   const int64_t rest = nt % 256;
-  const double tile_us = 2.0 * BM * BN * (double)p.T / CU_FLOPS;
-  g.S = 1;
-  double best = rest ? tile_us : 0.0;
-  for (int S = 2; S <= 16 && rest && p.T / S >= 64; S++) {
-    const double us = tile_us * (double)((rest * S + 255) / 256) / S + 4.0 + (double)(rest * S * BM * BN * 2 * sizeof(T)) / 3e6;
-    if (us < best) { best = us; g.S = S; }
-  }
+  g.S = tile_parts<T>(rest, BM, BN, p.T);
   g.part = nullptr;
   if (g.S > 1) {
     g.kc = ((p.T + g.S - 1) / g.S + TILE_K<T> - 1) / TILE_K<T> * TILE_K<T>;
@@ -163,19 +171,54 @@ static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hip
   return e;
 }
 
+// 32 wide along a side where that saves a sixth of the padded width or more
+static bool tile_narrow(int64_t n) { return 6 * ((n + 31) / 32 * 32) <= 5 * ((n + 63) / 64 * 64); }
+
 template <class T> static hipError_t tile_T(const MmPlan &p, const T *a, const T *b, T *c, hipStream_t s) {
   // a side below 8 fills too little of a 16-wide instruction, fewer k too
   // little of a stage (double, 10 x 4 x 100, 3000 of them: 23.6 us, the SIMT
   // kernel 21.2)
   if (p.H < 8 || p.W < 8 || p.T < 8) return hipErrorNotSupported;
-  // 32 wide along a side where that saves a sixth of the padded width or more
-  auto narrow = [](int64_t n) { return 6 * ((n + 31) / 32 * 32) <= 5 * ((n + 63) / 64 * 64); };
-  if (narrow(p.H)) {
-    if (narrow(p.W)) return tile_launch<T, 32, 32, 2, 2>(p, a, b, c, s);
+  if (tile_narrow(p.H)) {
+    if (tile_narrow(p.W)) return tile_launch<T, 32, 32, 2, 2>(p, a, b, c, s);
     return tile_launch<T, 32, 64, 1, 4>(p, a, b, c, s);
   }
-  if (narrow(p.W)) return tile_launch<T, 64, 32, 4, 1>(p, a, b, c, s);
+  if (tile_narrow(p.W) || p.variant == 32) return tile_launch<T, 64, 32, 4, 1>(p, a, b, c, s);
   return tile_launch<T, 64, 64, 2, 2>(p, a, b, c, s);
+}
+
+// Which engine runs a float product in the default mode: by its sizes alone, so
+// that its bits depend neither on a timing nor on what ran before.  Batches
+// have the kernel for 33..64 per side or the tiles, single products the tiles
+// where they are estimated to take no longer than the FP16 split, in us:
+//   tiles  15 + operations / 92e6 + outputs / 2.2e6
+//   split  50 + packed elements / 0.42e6 + outputs / 0.48e6 (stored, marked
+//          and looked over), and 0.0175 per k for each 256 blocks of 128x128
+// fitted to 140 products of 1.5e9 to 3e10 operations (standard deviations 10%
+// and 8%; the choice is the faster engine's but for 2% to 9% on 8 of them).
+// 1000^3: 31 and 69 us, 1587^3: 95 and 98, 2048^3: 170 and 115; 1000 x 6000 x
+// 700: 105 and 165, 2500 x 1000 x 2500: 139 and 95.  Beyond 3e10 operations
+// the split wins wherever it has blocks for the chip.
+constexpr double TILE_FLOPS = 8e9, SPLIT_FLOPS = 3e10;
+bool tile_takes_f32(const MmPlan &p) {
+  if (small_split16(p)) return false;
+  const double h = (double)p.H, w = (double)p.W, k = (double)p.T, flops = 2.0 * h * w * k;
+  if (!single_split16(p)) return p.nbatch != 1 || flops <= TILE_FLOPS;
+  if (flops > SPLIT_FLOPS) return false;
+  const int64_t waves = ((p.H + 127) / 128 * ((p.W + 127) / 128) + 255) / 256;
+  return 15 + flops / 92e6 + h * w / 2.2e6 <= 50 + (h + w) * k / 0.42e6 + h * w / 0.48e6 + 0.0175 * k * (double)waves;
+}
+
+// The widths of tile (MmPlan::variant) that the autotuner may choose from: 64
+// and, where neither width is cut along t and so both sum every output alike,
+// 64x32, which fills the chip better (600^3: 14 us against 21, 512^3: 12
+// against 14) and reads more (3173 x 76 x 4691: 59 against 52).
+std::vector<int> tile_widths_f32(const MmPlan &p) {
+  const int64_t n32 = (p.H + 63) / 64 * ((p.W + 31) / 32), n64 = (p.H + 63) / 64 * ((p.W + 63) / 64);
+  if (p.nbatch == 1 && !tile_narrow(p.H) && !tile_narrow(p.W) && tile_parts<float>(n64 % 256, 64, 64, p.T) == 1 &&
+      tile_parts<float>(n32 % 256, 64, 32, p.T) == 1)
+    return {64, 32};
+  return {64};
 }
 
 hipError_t launch_tile_f64(const MmPlan &p, const double *a, const double *b, double *c, hipStream_t s) {
