@@ -73,12 +73,11 @@ __global__ __launch_bounds__(256) void mm_simt(const T *__restrict__ a, const T 
                                                MmPlan p, int64_t ntm, int64_t ntn, int a_tfast, int b_wfast) {
   __shared__ T As[SB_K][SB_M + 1];
   __shared__ T Bs[SB_K][SB_N + 1];
-  int64_t blk = grid_block();
+  int64_t blk = blockIdx.x;
   const int64_t tm = blk % ntm;
   blk /= ntm;
   const int64_t tn = blk % ntn;
   const int64_t bidx = blk / ntn;
-  if (bidx >= p.nbatch) return;
   int64_t o[3];
   mm_batch_offsets(p, bidx, o);
   const int tid = threadIdx.x;
@@ -144,6 +143,32 @@ static hipError_t matmult_T(const MmPlan &p, const void *va, const void *vb, voi
   T *c = (T *)vc;
   const int64_t total = p.H * p.W * p.nbatch;
   if (total == 0) return hipSuccess;
+  // more blocks (of 32x32 or more each) than a grid holds: two launches of
+  // half the longest batch dim, or half the rows or columns
+  if (!bad && (p.H + 31) / 32 * ((p.W + 31) / 32) * p.nbatch >= GRID_BLOCKS / 2) {
+    MmPlan lo = p, hi = p;
+    int d = 0;
+    for (int k = 1; k < p.nd; k++) d = p.dims[k] > p.dims[d] ? k : d;
+    if (p.nbatch > 1) {
+      lo.dims[d] = p.dims[d] / 2;
+      hi.dims[d] = p.dims[d] - lo.dims[d];
+      lo.nbatch = p.nbatch / p.dims[d] * lo.dims[d];
+      hi.nbatch = p.nbatch - lo.nbatch;
+      for (int q = 0; q < 3; q++) hi.off[q] += lo.dims[d] * p.inc[q][d];
+    } else if (p.H >= p.W) {
+      lo.H = p.H / 128 * 64;
+      hi.H = p.H - lo.H;
+      hi.off[0] += lo.H * p.a_h;
+      hi.off[2] += lo.H * p.c_h;
+    } else {
+      lo.W = p.W / 128 * 64;
+      hi.W = p.W - lo.W;
+      hi.off[1] += lo.W * p.b_w;
+      hi.off[2] += lo.W * p.c_w;
+    }
+    const hipError_t e = matmult_T<T>(lo, va, vb, vc, bad, bi, mode, s);
+    return e == hipSuccess ? matmult_T<T>(hi, va, vb, vc, bad, bi, mode, s) : e;
+  }
   if (bad) {
     int64_t blocks = (total + 255) / 256;
     if (blocks > 65536) blocks = 65536;
@@ -169,8 +194,7 @@ static hipError_t matmult_T(const MmPlan &p, const void *va, const void *vb, voi
   }
   const int64_t ntm = (p.H + SB_M - 1) / SB_M, ntn = (p.W + SB_N - 1) / SB_N;
   const int64_t blocks = ntm * ntn * p.nbatch;
-  if (blocks >= ((int64_t)1 << 31)) return hipErrorInvalidConfiguration;
-  const dim3 grid = grid_of(blocks);
+  const dim3 grid((unsigned)blocks);
   const int a_tfast = (p.a_t == 1 || p.a_h != 1) ? 1 : 0;
   const int b_wfast = (p.b_w == 1 || p.b_t != 1) ? 1 : 0;
   const bool fused = IsFloat<T>::v && mode != PDLHIP_MM_PDLORDER;

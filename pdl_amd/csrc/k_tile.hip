@@ -39,7 +39,6 @@ template <class T> struct TilePlan {
   MmPlan p;
   int64_t ntm, ntn;    // tiles of one product
   int64_t nwhole;      // tiles summed over all of t; the others in S parts of kc
-  int64_t nblocks;
   int32_t S;
   int64_t kc;
   T *part;
@@ -73,8 +72,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && !FINE ? 3 : 4) void tile_gem
   const MmPlan &p = g.p;
   // whole tiles first, each XCD (block b runs on XCD b % 8) a contiguous
   // share of them, then the parts
-  int64_t t = grid_block(), kb = 0, ke = p.T;
-  if (t >= g.nblocks) return;
+  int64_t t = blockIdx.x, kb = 0, ke = p.T;
   int part = -1;
   if (t < g.nwhole) {
     if (g.nwhole % 8 == 0) t = (t % 8) * (g.nwhole / 8) + t / 8;
@@ -135,7 +133,7 @@ static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hip
   g.ntm = (p.H + BM - 1) / BM;
   g.ntn = (p.W + BN - 1) / BN;
   const int64_t nt = g.ntm * g.ntn * p.nbatch;
-  if (nt >= ((int64_t)1 << 30)) return hipErrorNotSupported;
+  if (nt >= GRID_BLOCKS / 2) return hipErrorNotSupported;   // (its parts are fewer than as many again)
   const int64_t rest = nt % 256;
   g.S = tile_parts<T>(rest, BM, BN, p.T);
   g.part = nullptr;
@@ -148,8 +146,7 @@ static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hip
   g.nwhole = g.S > 1 ? nt - rest : nt;
   if (g.S == 1) g.kc = p.T;
   const bool ak = p.a_t == 1, bk = p.b_t == 1;
-  g.nblocks = g.nwhole + (nt - g.nwhole) * g.S;
-  const dim3 grid = grid_of(g.nblocks);
+  const dim3 grid((unsigned)(g.nwhole + (nt - g.nwhole) * g.S));
   // (float) sums of 8 k rather than 32 where all of t is three stages or less
   auto go = [&](auto fine) {
     constexpr bool F = decltype(fine)::value;
@@ -189,8 +186,10 @@ template <class T> static hipError_t tile_T(const MmPlan &p, const T *a, const T
 
 // Which engine runs a float product in the default mode: by its sizes alone, so
 // that its bits depend neither on a timing nor on what ran before.  Batches
-// have the kernel for 33..64 per side or the tiles, single products the tiles
-// where they are estimated to take no longer than the FP16 split, in us:
+// have the kernel for 33..64 per side or the tiles; single products the tiles
+// where the FP16 split's 128x128 blocks do not fit (a side below 64 or fewer
+// than 32 k: @@) or where they
+// are estimated to take no longer than the split, in us:
 //   tiles  15 + operations / 92e6 + outputs / 2.2e6
 //   split  50 + packed elements / 0.42e6 + outputs / 0.48e6 (stored, marked
 //          and looked over), and 0.0175 per k for each 256 blocks of 128x128
@@ -199,11 +198,11 @@ template <class T> static hipError_t tile_T(const MmPlan &p, const T *a, const T
 // 1000^3: 31 and 69 us, 1587^3: 95 and 98, 2048^3: 170 and 115; 1000 x 6000 x
 // 700: 105 and 165, 2500 x 1000 x 2500: 139 and 95.  Beyond 3e10 operations
 // the split wins wherever it has blocks for the chip.
-constexpr double TILE_FLOPS = 8e9, SPLIT_FLOPS = 3e10;
+constexpr double SPLIT_FLOPS = 3e10;
 bool tile_takes_f32(const MmPlan &p) {
   if (small_split16(p)) return false;
   const double h = (double)p.H, w = (double)p.W, k = (double)p.T, flops = 2.0 * h * w * k;
-  if (!single_split16(p)) return p.nbatch != 1 || flops <= TILE_FLOPS;
+  if (!single_split16(p)) return true;
   if (flops > SPLIT_FLOPS) return false;
   const int64_t waves = ((p.H + 127) / 128 * ((p.W + 127) / 128) + 255) / 256;
   return 15 + flops / 92e6 + h * w / 2.2e6 <= 50 + (h + w) * k / 0.42e6 + h * w / 0.48e6 + 0.0175 * k * (double)waves;

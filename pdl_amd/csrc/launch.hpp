@@ -10,14 +10,15 @@ namespace pdlhip {
 
 // A launch dimension holds fewer than 2^32 threads: more wrap without an
 // error and the blocks past them never run.  In one dimension that is fewer
-// than GRID_BLOCKS blocks of 256 threads; grid_of lays out up to 2^31 - 1 of
-// them, block grid_block() of which is past the last one for a few.
+// than GRID_BLOCKS blocks of 256 threads; from there on grid_of lays them out
+// in rows of 2^20, the last of which runs past the last block.
 constexpr int64_t GRID_BLOCKS = (int64_t)1 << 24;
+constexpr int GRID_ROW = 20;
 inline dim3 grid_of(int64_t blocks) {
-  const int64_t ny = (blocks + (GRID_BLOCKS >> 1) - 1) / (GRID_BLOCKS >> 1);
-  return ny <= 1 ? dim3((unsigned)blocks) : dim3((unsigned)((blocks + ny - 1) / ny), (unsigned)ny);
+  if (blocks < GRID_BLOCKS) return dim3((unsigned)blocks);
+  return dim3(1u << GRID_ROW, (unsigned)((blocks + (1 << GRID_ROW) - 1) >> GRID_ROW));
 }
-__device__ __forceinline__ int64_t grid_block() { return (int64_t)blockIdx.y * gridDim.x + blockIdx.x; }
+__device__ __forceinline__ int64_t grid_block() { return ((int64_t)blockIdx.y << GRID_ROW) + blockIdx.x; }
 
 #define PDLHIP_FOR_EACH_TYPE(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
 

@@ -70,6 +70,17 @@ def test_batch_of_split16_products():
         assert bool((part == want).all())
 
 
+def test_one_product_of_many_tiles():
+    h, w = (1 << 18) + 5, (1 << 18) + 3     # 64 GiB of bytes
+    a, b = filled(C.L.B, [1, h], 0, 256, 7), filled(C.L.B, [w, 1], 0, 256, 8)
+    c = C.matmult(a, b)
+    assert c.dims == [w, h]
+    C.synchronize()
+    tb = tensor(b)
+    for pa, pc in zip(tensor(a).split(1 << 12), tensor(c).split(1 << 12)):
+        assert torch.equal(pc, pa * tb)
+
+
 def test_rows_of_a_broadcast():
     rows = (1 << 24) + 5
     a, b = filled(C.L.B, [128, rows], 0, 256, 5), filled(C.L.B, [128], 0, 256, 6)
