@@ -186,8 +186,10 @@ template <class T> static hipError_t tile_T(const MmPlan &p, const T *a, const T
 
 // Which engine runs a float product in the default mode: by its sizes alone, so
 // that its bits depend neither on a timing nor on what ran before.  Batches
-// have the kernel for 33..64 per side or the tiles, single products the tiles
-// where they are estimated to take no longer than the FP16 split, in us:
+// have the kernel for 33..64 per side or the tiles; single products the tiles
+// where the FP16 split's 128x128 blocks do not fit (a side below 64, or fewer
+// than 32 k; 32 x 20000 x 20000 takes 395 us, on the SIMT kernel 4380), or
+// where they are estimated to take no longer than the split, in us:
 //   tiles  15 + operations / 92e6 + outputs / 2.2e6
 //   split  50 + packed elements / 0.42e6 + outputs / 0.48e6 (stored, marked
 //          and looked over), and 0.0175 per k for each 256 blocks of 128x128
@@ -196,11 +198,11 @@ template <class T> static hipError_t tile_T(const MmPlan &p, const T *a, const T
 // 1000^3: 31 and 69 us, 1587^3: 95 and 98, 2048^3: 170 and 115; 1000 x 6000 x
 // 700: 105 and 165, 2500 x 1000 x 2500: 139 and 95.  Beyond 3e10 operations
 // the split wins wherever it has blocks for the chip.
-constexpr double TILE_FLOPS = 8e9, SPLIT_FLOPS = 3e10;
+constexpr double SPLIT_FLOPS = 3e10;
 bool tile_takes_f32(const MmPlan &p) {
   if (small_split16(p)) return false;
   const double h = (double)p.H, w = (double)p.W, k = (double)p.T, flops = 2.0 * h * w * k;
-  if (!single_split16(p)) return p.nbatch != 1 || flops <= TILE_FLOPS;
+  if (!single_split16(p)) return true;
   if (flops > SPLIT_FLOPS) return false;
   const int64_t waves = ((p.H + 127) / 128 * ((p.W + 127) / 128) + 255) / 256;
   return 15 + flops / 92e6 + h * w / 2.2e6 <= 50 + (h + w) * k / 0.42e6 + h * w / 0.48e6 + 0.0175 * k * (double)waves;
