@@ -64,11 +64,11 @@ __device__ inline void tile_at(const TilePlan<T> &g, int64_t t, int64_t *o, int6
   }
 }
 
-template <class T, int BM, int BN, int WR, int WC, bool AK, bool BK, bool FINE>
-__global__ __launch_bounds__(256, sizeof(T) == 4 && !FINE ? 3 : 4) void tile_gemm(const T *__restrict__ a, const T *__restrict__ b, T *__restrict__ c,
+template <class T, int BM, int BN, int WR, int WC, bool AK, bool BK, int HOW>
+__global__ __launch_bounds__(256, sizeof(T) == 4 && HOW == BY_STAGE ? 3 : 4) void tile_gemm(const T *__restrict__ a, const T *__restrict__ b, T *__restrict__ c,
                                                     TilePlan<T> g) {
-  __shared__ __align__(16) T sA[2][BM][TILE_P<T>];
-  __shared__ __align__(16) T sB[2][BN][TILE_P<T>];
+  __shared__ __align__(16) T sA[TILE_BUFS<HOW>][BM][TILE_P<T>];
+  __shared__ __align__(16) T sB[TILE_BUFS<HOW>][BN][TILE_P<T>];
   const MmPlan &p = g.p;
   // whole tiles first, each XCD (block b runs on XCD b % 8) a contiguous
   // share of them, then the parts
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256, sizeof(T) == 4 && !FINE ? 3 : 4) void tile_gem
   T *dst = part >= 0 ? g.part + ((t - g.nwhole) * g.S + part) * (BM * BN) : c + o[2] + n0 * p.c_w + m0 * p.c_h;
   const int64_t dh = part >= 0 ? BN : p.c_h, dw = part >= 0 ? 1 : p.c_w;
   const int64_t rows = part >= 0 ? BM : p.H - m0, cols = part >= 0 ? BN : p.W - n0;
-  tile_product<T, BM, BN, WR, WC, AK, BK, FINE>(a + o[0], b + o[1], p.H, p.W, p.a_h, p.a_t, p.b_w, p.b_t, m0, n0, kb, ke, sA,
+  tile_product<T, BM, BN, WR, WC, AK, BK, HOW>(a + o[0], b + o[1], p.H, p.W, p.a_h, p.a_t, p.b_w, p.b_t, m0, n0, kb, ke, sA,
                                           sB, [&](int h, int w, T v) {
                                             if (h < rows && w < cols) dst[h * dh + w * dw] = v;
                                           });
@@ -147,19 +147,25 @@ static hipError_t tile_launch(const MmPlan &p, const T *a, const T *b, T *c, hip
   if (g.S == 1) g.kc = p.T;
   const bool ak = p.a_t == 1, bk = p.b_t == 1;
   const dim3 grid((unsigned)(g.nwhole + (nt - g.nwhole) * g.S));
-  // (float) sums of 8 k rather than 32 where all of t is three stages or less
-  auto go = [&](auto fine) {
-    constexpr bool F = decltype(fine)::value;
+  // (float) sums of 8 k rather than 32 where all of t is three stages or less;
+  // up to half a stage, with the registers and LDS of that alone: eight blocks
+  // per CU instead of four and half the matrix instructions (2000 products of
+  // 100 x 8 x 100: 33 us against 50, 39 on the SIMT kernel, which also errs
+  // 10% more; 20000 of 40 x 8 x 40: 64, 111 and 72; one of 15000 x 8 x 15000:
+  // 232, 336 and 390)
+  auto go = [&](auto how) {
+    constexpr int F = decltype(how)::value;
     if (ak && bk) hipLaunchKernelGGL((tile_gemm<T, BM, BN, WR, WC, true, true, F>), grid, dim3(256), 0, s, a, b, c, g);
     else if (ak) hipLaunchKernelGGL((tile_gemm<T, BM, BN, WR, WC, true, false, F>), grid, dim3(256), 0, s, a, b, c, g);
     else if (bk) hipLaunchKernelGGL((tile_gemm<T, BM, BN, WR, WC, false, true, F>), grid, dim3(256), 0, s, a, b, c, g);
     else hipLaunchKernelGGL((tile_gemm<T, BM, BN, WR, WC, false, false, F>), grid, dim3(256), 0, s, a, b, c, g);
   };
   if constexpr (sizeof(T) == 4) {
-    if (p.T <= 96) go(std::true_type());
-    else go(std::false_type());
+    if (p.T <= TILE_K<T> / 2) go(std::integral_constant<int, HALF_STAGE>());
+    else if (p.T <= 96) go(std::integral_constant<int, BY_EIGHT>());
+    else go(std::integral_constant<int, BY_STAGE>());
   } else {
-    go(std::false_type());
+    go(std::integral_constant<int, BY_STAGE>());
   }
   if (g.part)
     hipLaunchKernelGGL((tile_join<T, BM, BN>), dim3((unsigned)((nt - g.nwhole) * (BM * BN / 256))), dim3(256), 0, s, c, g);

@@ -97,9 +97,14 @@ template <class T, int N, bool KFAST> struct TileLoad {
   }
 };
 
+// how a tile sums: a stage's k at a time (double: one chain), 8 k at a time
+// (float), or 8 k at a time where all of k is half a stage or less
+constexpr int BY_STAGE = 0, BY_EIGHT = 1, HALF_STAGE = 2;
+template <int HOW> constexpr int TILE_BUFS = HOW == HALF_STAGE ? 1 : 2;   // stages in LDS
+
 // the tile at (m0, n0) summed over k in [kb, ke), ke > kb; put(row, column,
 // value) for each of the thread's outputs, counted within the tile
-template <class T, int BM, int BN, int WR, int WC, bool AK, bool BK, bool FINE, class Put>
+template <class T, int BM, int BN, int WR, int WC, bool AK, bool BK, int HOW, class Put>
 __device__ __forceinline__ void tile_product(const T *a, const T *b, int64_t H, int64_t W, int64_t a_h, int64_t a_t,
                                              int64_t b_w, int64_t b_t, int64_t m0, int64_t n0, int64_t kb, int64_t ke,
                                              T (*sA)[BM][TILE_P<T>], T (*sB)[BN][TILE_P<T>], Put put) {
@@ -139,7 +144,7 @@ __device__ __forceinline__ void tile_product(const T *a, const T *b, int64_t H, 
   };
   // Double: one chain of sums per output.  Float: the matrix cores round at
   // every k, so a few k at a time are summed from zero and their sum added to
-  // the total: a stage's 32 k, or 8 where there are few (FINE).  The error of
+  // the total: a stage's 32 k, or 8 where there are few.  The error of
   // 1024^3 is then 1.5e-7 instead of 5.7e-7, of 64^3 8e-8 instead of 1.5e-7
   // (the FP16 split's: 3.5e-7 and 9e-8); the adds run on the vector unit
   // while the matrix cores go on with the other tiles.
@@ -158,7 +163,7 @@ __device__ __forceinline__ void tile_product(const T *a, const T *b, int64_t H, 
           if constexpr (sizeof(T) == 8) {
             acc[i][j] = TT::mfma(af[half][i][u], bf[half][j][u], acc[i][j]);
           } else {
-            const bool fresh = FINE ? u % 2 == 0 : half == 0 && u == 0;
+            const bool fresh = HOW != BY_STAGE ? u % 2 == 0 : half == 0 && u == 0;
             if (fresh) acc[i][j] += part[i][j];
             part[i][j] = TT::mfma(af[half][i][u], bf[half][j][u], fresh ? typename TT::acc_t{} : part[i][j]);
           }
@@ -181,22 +186,26 @@ __device__ __forceinline__ void tile_product(const T *a, const T *b, int64_t H, 
     multiply(0);
     multiply(1);
   };
-  if (n > 1) {
+  if (HOW != HALF_STAGE && n > 1) {
     fetch(1, 1);
     fetch(0, 2);
   }
   __syncthreads();
   frags(0, 0);
-  int64_t q = 0;
-  for (; q + 2 < n; q += 2) {
-    step(0, q);
-    step(1, q + 1);
-  }
-  if (q + 1 < n) {
-    step(0, q);
-    last_step(1);
+  if constexpr (HOW == HALF_STAGE) {
+    multiply(0);
   } else {
-    last_step(0);
+    int64_t q = 0;
+    for (; q + 2 < n; q += 2) {
+      step(0, q);
+      step(1, q + 1);
+    }
+    if (q + 1 < n) {
+      step(0, q);
+      last_step(1);
+    } else {
+      last_step(0);
+    }
   }
   if constexpr (sizeof(T) == 4) {
 #pragma unroll
