@@ -263,7 +263,9 @@ pdlhip_error pdlhip_op_info(const char *op, int *npdls, int *nparents);
  * reference counterpart: PDL runs such a list as a Perl loop of matmult
  * calls.  mode PDLHIP_LIST_QUEUE: one persistent launch over a device list of
  * (product, tile) items, largest inner dimension first, kernel and tile shape
- * picked per shape class by a timing autotuner and cached; PDLHIP_LIST_EACH:
+ * picked per shape class by a timing autotuner and cached (a second launch
+ * for products of another layout than most, or of an inner dimension below
+ * one 16-byte load); PDLHIP_LIST_EACH:
  * one launch per product (the comparison point).  Items that need a type
  * conversion or bad-value handling run through pdlhip_run_matmult. */
 enum { PDLHIP_LIST_QUEUE = 0, PDLHIP_LIST_EACH = 1 };
@@ -272,7 +274,7 @@ pdlhip_error pdlhip_run_matmult_list(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlh
 /* A prepared matmult list (no reference counterpart): the entries are
  * planned once as pdlhip_run_matmult_list plans them (outputs created),
  * their items and tile decompositions kept in HBM; each launch then runs
- * the whole list (PDLHIP_LIST_QUEUE: one persistent launch,
+ * the whole list (PDLHIP_LIST_QUEUE: one persistent launch or two,
  * PDLHIP_LIST_EACH: one launch per product) and allocates nothing, so it can
  * be captured in a HIP graph.  Entries with bad values, needing a type
  * conversion or of another type than the first are refused. */

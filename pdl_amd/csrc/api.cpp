@@ -25,6 +25,7 @@
 #include <functional>
 #include <map>
 #include <mutex>
+#include <numeric>
 #include <queue>
 #include <string>
 #include <tuple>
@@ -1484,7 +1485,7 @@ static pdlhip_error run(const Sig &s, pdlhip_pdl **user, int npdls, const int64_
 // Measured choices of kernel variants per shape class, kept in a text file
 // per GPU architecture so that later processes reuse them: one line per
 // entry, "<key> <choice>", the key naming the kernel family, element type,
-// shape class and architecture (e.g. "list:float:tiles1:dim2^8:items2^12:gfx950").
+// shape class and architecture (e.g. "list:float:tiles1:form1:fused1:dim2^8:items2^12:gfx950").
 // The file is $PDLHIP_TUNE_FILE, else $XDG_CACHE_HOME/pdlhip/tune-<arch>.txt,
 // else $HOME/.cache/pdlhip/tune-<arch>.txt; PDLHIP_TUNE=0 turns timing off
 // (each family's default rule applies), PDLHIP_TUNE_VERBOSE=1 prints each
@@ -1581,16 +1582,28 @@ static int ilog2(int64_t v) {
   return r;
 }
 
+struct ListWork {
+  std::vector<int3> items;
+  unsigned longest = 0;   // of the bins
+  int3 *dev = nullptr;
+};
+// The matrix-core kernel loads by 16 bytes along k where every product it is
+// given allows that for an operand.  The products of a list that do not allow
+// what most of its work does (a shorter inner dimension, another layout) are
+// a part of their own, with a launch of its own: one product of inner
+// dimension 1 among 2000 floats of 8..256 a side made the whole list take 395
+// us instead of 273 (now 286; with every tenth operand transposed 385, now 295).
+enum { LIST_ALL, LIST_MOST, LIST_REST, LIST_PARTS };
 // A planned matmult list: the items (one product per broadcast position of
 // every list entry) and both tile decompositions in HBM, the tile picked by
 // the autotuner.  A launch allocates nothing.
 struct ListH {
   Deferred d;
-  std::vector<int3> work32, work64;
+  ListWork work[LIST_PARTS][2];   // work items of 64x64, 32x32
+  int form = 0, rest_form = 0;    // list_form of LIST_MOST and of LIST_REST, which are empty
+  bool mixed = false;             // where all products take one form
   MmItem *d_items = nullptr;
   unsigned int *d_counter = nullptr;
-  int3 *d_w32 = nullptr, *d_w64 = nullptr;
-  unsigned long32 = 0, long64 = 0;   // work items of the longest bin
   int tile = 64;        // 32 / 64: SIMT tiles; 0 / 2: the matrix cores, 64x64 / 32x32 work items; 1: BF16 split
   bool mfma = false;    // float/double list in a default mode whose items fit 32-bit offsets
 };
@@ -1598,17 +1611,27 @@ struct ListH {
 static void list_release(ListH &h) {
   dev_free(h.d_items);
   dev_free(h.d_counter);
-  dev_free(h.d_w32);
-  dev_free(h.d_w64);
-  h.d_items = nullptr; h.d_counter = nullptr; h.d_w32 = nullptr; h.d_w64 = nullptr;
+  h.d_items = nullptr; h.d_counter = nullptr;
+  for (auto &part : h.work)
+    for (ListWork &w : part) {
+      dev_free(w.dev);
+      w.dev = nullptr;
+    }
 }
 
+// the device block: 8 bin counters 128 bytes apart, then each work list's bounds
+static unsigned list_bounds(int part, int small) { return 256 + (unsigned)(2 * part + small) * 9; }
+
 static hipError_t list_launch(const ListH &h, int tile, bool each) {
-  const bool small = tile == 32 || tile == 2;
-  const std::vector<int3> &w = small ? h.work32 : h.work64;
-  const int nblocks = (int)std::max<size_t>(std::min<size_t>(w.size(), 2048), 1);
-  return launch_matmult_list(h.d.T, h.d_items, h.d.items.data(), (int)h.d.items.size(), small ? h.d_w32 : h.d_w64,
-                             (unsigned)w.size(), small ? h.long32 : h.long64, h.d_counter, tile, h.d.fused, each, nblocks, g.stream);
+  const int small = tile == 32 || tile == 2;
+  const ListWork &w = h.work[LIST_ALL][small];
+  const int nblocks = (int)std::max<size_t>(std::min<size_t>(w.items.size(), 2048), 1);
+  auto part = [&](int p, int form) {
+    return ListPart{h.work[p][small].dev, h.d_counter + list_bounds(p, small), h.work[p][small].longest, form};
+  };
+  const ListPart parts[2] = {part(h.mixed ? LIST_MOST : LIST_ALL, h.form), part(LIST_REST, h.rest_form)};
+  return launch_matmult_list(h.d.T, h.d_items, h.d.items.data(), (int)h.d.items.size(), w.dev, h.d_counter, parts,
+                             h.mixed ? 2 : 1, tile, h.d.fused, each, nblocks, g.stream);
 }
 
 // plan every entry through pdl_run_matmult's checks (outputs created as
@@ -1643,10 +1666,11 @@ static pdlhip_error list_build(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlhip_pdl
   // 8 bins, one per XCD (the kernels' list_next): each product, largest
   // inner dimension first, goes whole to the bin with the least work so far
   // (tiles x k); the bins lie back to back, bounds[x] .. bounds[x + 1]
-  auto build_work = [&](int tile, std::vector<int3> &work, unsigned *bounds, unsigned &longest) {
+  auto build_work = [&](int tile, ListWork &w, unsigned *bounds, auto in) {
     std::vector<std::vector<int3>> bins(8);
     std::vector<double> load(8, 0.0);
     for (int i : order) {
+      if (!in(i)) continue;
       const MmItem &it = h.d.items[i];
       int64_t ntm = (it.H + tile - 1) / tile, ntn = (it.W + tile - 1) / tile;
       const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
@@ -1654,19 +1678,45 @@ static pdlhip_error list_build(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlhip_pdl
       for (int64_t tm = 0; tm < ntm; tm++)
         for (int64_t tn = 0; tn < ntn; tn++) bins[x].push_back(make_int3(i, (int)tm, (int)tn));
     }
-    work.clear();
+    w.items.clear();
     for (int x = 0; x < 8; x++) {
-      bounds[x] = (unsigned)work.size();
-      work.insert(work.end(), bins[x].begin(), bins[x].end());
-      longest = std::max(longest, (unsigned)bins[x].size());
+      bounds[x] = (unsigned)w.items.size();
+      w.items.insert(w.items.end(), bins[x].begin(), bins[x].end());
+      w.longest = std::max(w.longest, (unsigned)bins[x].size());
     }
-    bounds[8] = (unsigned)work.size();
+    bounds[8] = (unsigned)w.items.size();
   };
-  // the device block: 8 bin counters 128 bytes apart, then the 64-tile
-  // list's bounds, then the 32-tile list's
-  unsigned qinit[256 + 9 + 9] = {0};
-  build_work(64, h.work64, qinit + 256, h.long64);
-  build_work(32, h.work32, qinit + 265, h.long32);
+  // the form that most of the work takes, and whether other products have less
+  std::vector<int> form(nit, 0);
+  double by_form[4] = {0, 0, 0, 0};
+  if (h.d.fused && (h.d.T == PDLHIP_F || h.d.T == PDLHIP_D))
+    for (int i = 0; i < nit; i++) {
+      const MmItem &it = h.d.items[i];
+      form[i] = list_form(h.d.T, it);
+      by_form[form[i]] += (double)it.H * (double)it.W * (double)std::max<int64_t>(it.T, 1);
+    }
+  h.form = (int)(std::max_element(by_form, by_form + 4) - by_form);
+  // (a list of fewer than 1.5e8 multiplications takes the form all products
+  // have: the second launch costs about 3 us, other loads a third of the time;
+  // 300 doubles of 8..64 a side with one of inner dimension 1: 9.7 us, 11.5 in
+  // two launches)
+  if (by_form[0] + by_form[1] + by_form[2] + by_form[3] < 1.5e8)
+    h.form = std::accumulate(form.begin(), form.end(), 3, [](int x, int y) { return x & y; });
+  auto most = [&](int i) { return (form[i] & h.form) == h.form; };
+  h.rest_form = 3;
+  for (int i = 0; i < nit; i++)
+    if (!most(i)) {
+      h.mixed = true;
+      h.rest_form &= form[i];
+    }
+  unsigned qinit[256 + 2 * LIST_PARTS * 9] = {0};
+  for (int small = 0; small < 2; small++) {
+    build_work(small ? 32 : 64, h.work[LIST_ALL][small], qinit + list_bounds(LIST_ALL, small), [](int) { return true; });
+    if (!h.mixed) continue;
+    build_work(small ? 32 : 64, h.work[LIST_MOST][small], qinit + list_bounds(LIST_MOST, small), most);
+    build_work(small ? 32 : 64, h.work[LIST_REST][small], qinit + list_bounds(LIST_REST, small),
+               [&](int i) { return !most(i); });
+  }
   // the matrix-core kernel indexes within a product with 32-bit offsets
   auto span = [](int64_t n1, int64_t i1, int64_t n2, int64_t i2) {
     return (n1 > 0 ? n1 - 1 : 0) * (i1 < 0 ? -i1 : i1) + (n2 > 0 ? n2 - 1 : 0) * (i2 < 0 ? -i2 : i2);
@@ -1678,16 +1728,21 @@ static pdlhip_error list_build(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlhip_pdl
       h.mfma = false;
   h.d_items = (MmItem *)dev_alloc(sizeof(MmItem) * nit);
   h.d_counter = (unsigned int *)dev_alloc(sizeof qinit);
-  h.d_w32 = (int3 *)dev_alloc(sizeof(int3) * std::max<size_t>(h.work32.size(), 1));
-  h.d_w64 = (int3 *)dev_alloc(sizeof(int3) * std::max<size_t>(h.work64.size(), 1));
-  if (!h.d_items || !h.d_counter || !h.d_w32 || !h.d_w64) {
+  bool got = h.d_items && h.d_counter;
+  for (auto &part : h.work)
+    for (ListWork &w : part) {
+      w.dev = (int3 *)dev_alloc(sizeof(int3) * std::max<size_t>(w.items.size(), 1));
+      got = got && w.dev;
+    }
+  if (!got) {
     list_release(h);
     return oom_err("matmult list");
   }
   hipError_t e = upload_now(h.d_items, h.d.items.data(), sizeof(MmItem) * nit);
   if (e == hipSuccess) e = upload_now(h.d_counter, qinit, sizeof qinit);
-  if (e == hipSuccess) e = upload_now(h.d_w32, h.work32.data(), sizeof(int3) * h.work32.size());
-  if (e == hipSuccess) e = upload_now(h.d_w64, h.work64.data(), sizeof(int3) * h.work64.size());
+  for (auto &part : h.work)
+    for (ListWork &w : part)
+      if (e == hipSuccess) e = upload_now(w.dev, w.items.data(), sizeof(int3) * w.items.size());
   // tile by the autotuner: 32 / 64 SIMT tiles, the FP32/FP64 matrix cores
   // with 64x64 (0) or 32x32 (2) work items and, for float, the BF16 three-way
   // split (1); timed on a copy of the item table whose outputs all point into
@@ -1698,8 +1753,8 @@ static pdlhip_error list_build(int n, pdlhip_pdl **a, pdlhip_pdl **b, pdlhip_pdl
     if (h.mfma && h.d.T == PDLHIP_F) cands.push_back(1);
     const int dflt = h.mfma ? 0 : 64;
     char fam[160];
-    snprintf(fam, sizeof fam, "list:%s:tiles%d:fused%d:dim2^%d:items2^%d", type_name(h.d.T), h.mfma ? 1 : 0,
-             h.d.fused ? 1 : 0, ilog2(maxdim), ilog2(nit));
+    snprintf(fam, sizeof fam, "list:%s:tiles%d:form%d:fused%d:dim2^%d:items2^%d", type_name(h.d.T), h.mfma ? 1 : 0,
+             h.form, h.d.fused ? 1 : 0, ilog2(maxdim), ilog2(nit));
     MmItem *t_items = nullptr;
     void *t_c = nullptr;
     auto run_one = [&](int cand) -> hipError_t {

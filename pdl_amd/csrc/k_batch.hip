@@ -565,7 +565,7 @@ __global__ __launch_bounds__(256) void list_bf16x3_one(const MmItem *__restrict_
 }
 
 static hipError_t list_bf16x3(const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
-                              unsigned int nwork, unsigned int *d_counter, bool each, int nblocks, hipStream_t s) {
+                              unsigned int *d_counter, bool each, int nblocks, hipStream_t s) {
   if (!each) {
     hipLaunchKernelGGL(list_reset, dim3(1), dim3(64), 0, s, d_counter);
     hipLaunchKernelGGL(list_bf16x3_queue, dim3(nblocks), dim3(256), 0, s, d_items, d_work,
@@ -580,44 +580,43 @@ static hipError_t list_bf16x3(const MmItem *d_items, const MmItem *h_items, int 
   return hipGetLastError();
 }
 
+template <class T> static int form_of(const MmItem &it) {
+  if (it.T == 0) return 3;                // loads nothing of its operands
+  const bool whole = it.T >= TILE_V<T>;   // as many k as one load takes
+  return (it.a_t == 1 && whole ? 1 : 0) | (it.b_t == 1 && whole ? 2 : 0);
+}
+int list_form(int T, const MmItem &it) { return T == PDLHIP_D ? form_of<double>(it) : form_of<float>(it); }
+
 template <class T, int TS>
-static hipError_t list_tiles_T(const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
-                               unsigned longest, unsigned int *d_counter, bool each, hipStream_t s) {
-  // 16-byte loads along k where every product has it unit-stride and as many
-  // k as one load takes
-  bool ak = true, bk = true;
-  for (int i = 0; i < nitems; i++) {
-    const bool whole = h_items[i].T >= TILE_V<T> || h_items[i].T == 0;
-    ak = ak && h_items[i].a_t == 1 && whole;
-    bk = bk && h_items[i].b_t == 1 && whole;
-  }
-  auto go = [&](unsigned grid, const int3 *work, int only, unsigned ntn) {
-    const unsigned int *bounds = (const unsigned int *)d_counter + LIST_BOUNDS + (TS == 32 ? LIST_BINS + 1 : 0);
-    if (ak && bk)
+static hipError_t list_tiles_T(const MmItem *d_items, const MmItem *h_items, int nitems, const ListPart *parts,
+                               int nparts, bool each, hipStream_t s) {
+  auto go = [&](int form, unsigned grid, const int3 *work, const unsigned int *bounds, int only, unsigned ntn) {
+    if (form == 3)
       hipLaunchKernelGGL((list_tiles<T, TS, true, true>), dim3(grid), dim3(256), 0, s, d_items, work, bounds, only, ntn);
-    else if (ak)
+    else if (form == 1)
       hipLaunchKernelGGL((list_tiles<T, TS, true, false>), dim3(grid), dim3(256), 0, s, d_items, work, bounds, only, ntn);
-    else if (bk)
+    else if (form == 2)
       hipLaunchKernelGGL((list_tiles<T, TS, false, true>), dim3(grid), dim3(256), 0, s, d_items, work, bounds, only, ntn);
     else
       hipLaunchKernelGGL((list_tiles<T, TS, false, false>), dim3(grid), dim3(256), 0, s, d_items, work, bounds, only, ntn);
   };
   if (!each) {   // as many blocks as are resident at once
-    go(LIST_BINS * std::min(std::max(longest, 1u), 32u * LIST_PER_CU<TS>), d_work, 0, 1);
+    for (int i = 0; i < nparts; i++)
+      go(parts[i].form, LIST_BINS * std::min(std::max(parts[i].longest, 1u), 32u * LIST_PER_CU<TS>), parts[i].work,
+         parts[i].bounds, 0, 1);
     return hipGetLastError();
   }
   for (int i = 0; i < nitems; i++) {
     const int64_t ntm = (h_items[i].H + TS - 1) / TS, ntn = (h_items[i].W + TS - 1) / TS;
     if (ntm * ntn == 0) continue;             // an empty k stores zeros
-    go((unsigned)(ntm * ntn), nullptr, i, (unsigned)ntn);
+    go(form_of<T>(h_items[i]), (unsigned)(ntm * ntn), nullptr, nullptr, i, (unsigned)ntn);
   }
   return hipGetLastError();
 }
 
 template <class T>
 static hipError_t list_T(const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
-                         unsigned int nwork, unsigned int *d_counter, int tile, bool fused, bool each, int nblocks,
-                         hipStream_t s) {
+                         unsigned int *d_counter, int tile, bool fused, bool each, int nblocks, hipStream_t s) {
 #define LQ(F, TS) hipLaunchKernelGGL((list_queue<T, F, TS>), dim3(nblocks), dim3(256), 0, s, d_items, d_work, \
                                      (const unsigned int *)d_counter + LIST_BOUNDS + (TS == 32 ? LIST_BINS + 1 : 0), \
                                      d_counter)
@@ -640,24 +639,24 @@ static hipError_t list_T(const MmItem *d_items, const MmItem *h_items, int nitem
 }
 
 hipError_t launch_matmult_list(int T, const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
-                               unsigned int nwork, unsigned int longest, unsigned int *d_counter, int tile, bool fused,
+                               unsigned int *d_counter, const ListPart *parts, int nparts, int tile, bool fused,
                                bool each, int nblocks, hipStream_t s) {
   // tile 0 / 2: the matrix-core kernels (64x64 / 32x32 work items), float and
   // double lists in the default modes; tile 1: float on the BF16 matrix cores
   if (tile == 1 && fused && T == PDLHIP_F)
-    return list_bf16x3(d_items, h_items, nitems, d_work, nwork, d_counter, each, nblocks, s);
+    return list_bf16x3(d_items, h_items, nitems, d_work, d_counter, each, nblocks, s);
   if (tile == 1) tile = 0;
   if (fused && T == PDLHIP_F && (tile == 0 || tile == 2))
-    return tile == 0 ? list_tiles_T<float, 64>(d_items, h_items, nitems, d_work, longest, d_counter, each, s)
-                     : list_tiles_T<float, 32>(d_items, h_items, nitems, d_work, longest, d_counter, each, s);
+    return tile == 0 ? list_tiles_T<float, 64>(d_items, h_items, nitems, parts, nparts, each, s)
+                     : list_tiles_T<float, 32>(d_items, h_items, nitems, parts, nparts, each, s);
   if (fused && T == PDLHIP_D && (tile == 0 || tile == 2))
-    return tile == 0 ? list_tiles_T<double, 64>(d_items, h_items, nitems, d_work, longest, d_counter, each, s)
-                     : list_tiles_T<double, 32>(d_items, h_items, nitems, d_work, longest, d_counter, each, s);
+    return tile == 0 ? list_tiles_T<double, 64>(d_items, h_items, nitems, parts, nparts, each, s)
+                     : list_tiles_T<double, 32>(d_items, h_items, nitems, parts, nparts, each, s);
   if (tile == 0) tile = 64;
   if (tile == 2) tile = 32;
   switch (T) {
-#define X(TC) case TC: return list_T<CType<TC>::T>(d_items, h_items, nitems, d_work, nwork, d_counter, tile, \
-                                                   fused, each, nblocks, s);
+#define X(TC) case TC: return list_T<CType<TC>::T>(d_items, h_items, nitems, d_work, d_counter, tile, fused, each, \
+                                                   nblocks, s);
     PDLHIP_FOR_EACH_TYPE(X)
 #undef X
   default: return hipErrorInvalidValue;

@@ -41,11 +41,25 @@ PDLHIP_FOR_EACH_TYPE(X)
 PDLHIP_FOR_EACH_TYPE(X)
 #undef X
 
-// a list of products in one persistent launch, or one launch per product
-// (each = true) (k_batch.hip); longest: work items of the longest of 8 bins
+// how the matrix-core list kernel can load a product's operands of type T: 1
+// A, 2 B in 16-byte loads along k (k_batch.hip)
+int list_form(int T, const MmItem &it);
+
+// products whose loads take one form: their work items in 8 bins, the bins'
+// bounds (device) and the longest bin's length
+struct ListPart {
+  const int3 *work;
+  const unsigned int *bounds;
+  unsigned int longest;
+  int form;
+};
+
+// a list of products in a persistent launch, of the queue d_work of all of
+// them or, on the matrix cores, of each part; or one launch per product (each
+// = true) (k_batch.hip)
 hipError_t launch_matmult_list(int T, const MmItem *d_items, const MmItem *h_items, int nitems, const int3 *d_work,
-                               unsigned int nwork, unsigned int longest, unsigned int *d_counter, int tile, bool fused, bool each,
-                               int nblocks, hipStream_t s);
+                               unsigned int *d_counter, const ListPart *parts, int nparts, int tile, bool fused,
+                               bool each, int nblocks, hipStream_t s);
 
 // Bad.pd elementwise ops (k_badops.hip): a of type T, mask int32 (setbadif),
 // b of type T (int32 for isbad/isgood); dval the double OtherPar; flag set
