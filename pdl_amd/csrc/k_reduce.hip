@@ -59,7 +59,7 @@ constexpr int RT = 256;  // threads per block (4 waves)
 // lane, then 16-byte vectors, then the rest one to a lane, each lane's in
 // increasing index order.  (Rows of odd length start unaligned; loading those
 // an element at a time took 167 us for 64 rows of 32091 ints.)
-template <int OP, class Tin, class Tacc, bool BAD, int NL>
+template <int OP, class Tin, class Tacc, bool BAD, int NL, bool ON16 = false>
 __device__ inline void row_segment(Part<Tin, Tacc> &pt, const Tin *__restrict__ row, int64_t begin, int64_t end,
                                    int lane, const BadInfo &ba, bool stream) {
   constexpr int VEC = 16 / sizeof(Tin);
@@ -67,13 +67,16 @@ __device__ inline void row_segment(Part<Tin, Tacc> &pt, const Tin *__restrict__ 
   // the narrower ones (eight or sixteen elements per load already)
   constexpr int RED_U = sizeof(Tin) >= 4 ? 4 : 2;
   const Tin abv = bv_as<Tin>(ba.bv);
-  const int64_t lead = ((16 - (int)((uintptr_t)(row + begin) & 15)) & 15) / sizeof(Tin);
+  const int64_t lead = ON16 ? 0 : ((16 - (int)((uintptr_t)(row + begin) & 15)) & 15) / sizeof(Tin);
   const int64_t vb = begin + lead < end ? begin + lead : end, ve = vb + (end - vb) / VEC * VEC;
+  // only floats have NaN for a bad value: without its test an element's mask is
+  // one compare (1000000 rows of 64 bytes with bad values: @@)
+  const int nan = IsFloat<Tin>::v ? ba.isnan : 0;
   auto push = [&](Tin x, int64_t i) {
-    if constexpr (BAD) { if (isbad(x, abv, ba.isnan)) return; }
+    if constexpr (BAD) { if (isbad(x, abv, nan)) return; }
     part_push<OP, Tin, Tacc>(pt, x, i);
   };
-  if (begin + lane < vb) push(row[begin + lane], begin + lane);
+  if (!ON16 && begin + lane < vb) push(row[begin + lane], begin + lane);
   int64_t i = vb + (int64_t)lane * VEC;
   for (; i + (RED_U - 1) * NL * VEC < ve; i += RED_U * NL * VEC) {
     Vec<Tin, VEC> x[RED_U];
@@ -110,7 +113,7 @@ __device__ inline void waves_join(Part<Tin, Tacc> &pt, Part<Tin, Tacc> *sh) {
 
 // NW waves per row; four rows per block of 256 threads for NW = 1, else a
 // row per block
-template <int OP, class Tin, class Tout, class Tacc, bool BAD, int NW>
+template <int OP, class Tin, class Tout, class Tacc, bool BAD, int NW, bool ON16 = false>
 __global__ __launch_bounds__(NW > 4 ? NW * 64 : RT) void red_wave(const Tin *__restrict__ a, RedPlan p, Outs o,
                                                                   BadInfo ba, bool stream) {
   constexpr int PER = NW == 1 ? 4 : 1;
@@ -121,7 +124,7 @@ __global__ __launch_bounds__(NW > 4 ? NW * 64 : RT) void red_wave(const Tin *__r
     out_offsets(p, e, off);
     Part<Tin, Tacc> pt;
     part_init<OP, Tin, Tacc>(pt);
-    row_segment<OP, Tin, Tacc, BAD, NW * 64>(pt, a + off[0], 0, p.n, NW == 1 ? lane : (int)threadIdx.x, ba, stream);
+    row_segment<OP, Tin, Tacc, BAD, NW * 64, ON16>(pt, a + off[0], 0, p.n, NW == 1 ? lane : (int)threadIdx.x, ba, stream);
     wave_reduce<OP, Tin, Tacc>(pt);
     if constexpr (NW > 1) {
       waves_join<OP, Tin, Tacc, NW>(pt, sh);
@@ -773,8 +776,14 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
       if (p.nout >= 4096 || loads < 8) {
         int64_t blocks = (p.nout + 3) / 4;
         if (blocks > 65536) blocks = 65536;
-        hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 1>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
-                           stream);
+        bool on16 = (uintptr_t)(a + p.off[0]) % 16 == 0;
+        for (int d = 0; d < p.nd; d++) on16 = on16 && p.inc[0][d] * (int64_t)sizeof(Tin) % 16 == 0;
+        if (on16)
+          hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 1, true>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p,
+                             o, ba, stream);
+        else
+          hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 1>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o,
+                             ba, stream);
       } else if (p.nout >= 1024 || loads < 32) {
         hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 4>), dim3((unsigned)p.nout), dim3(RT), 0, s, a, p, o, ba,
                            stream);
