@@ -59,6 +59,8 @@ constexpr int RT = 256;  // threads per block (4 waves)
 // lane, then 16-byte vectors, then the rest one to a lane, each lane's in
 // increasing index order.  (Rows of odd length start unaligned; loading those
 // an element at a time took 167 us for 64 rows of 32091 ints.)
+// ON16: every row starts on such a boundary, and a short one is spared the
+// search for it (1000000 rows of 64 floats: 346 us, 372 with it).
 template <int OP, class Tin, class Tacc, bool BAD, int NL, bool ON16 = false>
 __device__ inline void row_segment(Part<Tin, Tacc> &pt, const Tin *__restrict__ row, int64_t begin, int64_t end,
                                    int lane, const BadInfo &ba, bool stream) {
@@ -70,7 +72,7 @@ __device__ inline void row_segment(Part<Tin, Tacc> &pt, const Tin *__restrict__ 
   const int64_t lead = ON16 ? 0 : ((16 - (int)((uintptr_t)(row + begin) & 15)) & 15) / sizeof(Tin);
   const int64_t vb = begin + lead < end ? begin + lead : end, ve = vb + (end - vb) / VEC * VEC;
   // only floats have NaN for a bad value: without its test an element's mask is
-  // one compare (1000000 rows of 64 bytes with bad values: @@)
+  // one compare (1000000 rows of 64 bytes with bad values: 273 us, 335 with it)
   const int nan = IsFloat<Tin>::v ? ba.isnan : 0;
   auto push = [&](Tin x, int64_t i) {
     if constexpr (BAD) { if (isbad(x, abv, nan)) return; }
