@@ -16,7 +16,6 @@ Perl-level wrapper logic restated here (cited where defined):
 """
 import ctypes
 import struct
-import threading
 import weakref
 
 import numpy as np
@@ -1167,14 +1166,11 @@ class _Args:
         return self.run
 
 
-class _Spare(threading.local):
-    """A thread's argument block while no call has it.  A call takes it out
-    and puts it back: Python may run other code of the same thread in the
-    middle of one (a signal handler, a finalizer the garbage collector calls),
-    and an op in there finds no block and makes its own."""
-
-
-_spare = _Spare()
+# Argument blocks no call has.  A call takes one out and puts it back: another
+# thread, or other code of the same thread that Python runs in the middle of a
+# call (a signal handler, a finalizer the garbage collector calls), finds
+# another or makes its own.  (pop and append are atomic.)
+_spare = []
 
 
 def _pdl_struct(nd):
@@ -1192,60 +1188,59 @@ _STATE_AT, _DIMS_AT, _INCS_AT, _DATA_AT = (L.Pdl.state.offset, L.Pdl.dims.offset
 
 def _call(op, pdls, swap=0, m_size=None, dpar=None):
     """the bare C ABI call (no dataflow bookkeeping)"""
-    A = _spare.__dict__.pop("args", None) or _Args()
     try:
-        return _call_in(A, op, pdls, swap, m_size, dpar)
+        A = _spare.pop()
+    except IndexError:
+        A = _Args()
+    try:
+        n = len(pdls)
+        if n > A.MAX:
+            raise PDLError(L.EUSERERROR, "pdlhip: %s: %d ndarrays" % (op, n))
+        mem, table_at, o = A.mem, A.table_at, 0
+        for p in pdls:
+            dims, incs, buf = p.dims, p.incs, p._buf
+            nd = len(dims)
+            if nd > L.MAXDIMS:
+                raise PDLError(L.EUSERERROR, "too many dims")
+            if len(incs) != nd:
+                incs = incs[:nd]
+            _STRUCTS[nd].pack_into(mem, o, p.dtype, p.state, nd, 0, *dims, *incs, p.offs,
+                                   buf.ptr or 0 if buf is not None else 0)
+            if p.bids or p.badvalue_ is not None:
+                p._rest_to_c(A.pdls[o // A.size])
+            o += A.size
+        first = range(n)       # which struct each ndarray is: one passed twice is one pdl
+        if n > 1 and (pdls[0] is pdls[1] or n > 2 and len(set(map(id, pdls))) < n):
+            first = [next(j for j in range(n) if pdls[j] is p) for p in pdls]
+            for i in range(n):
+                A.shared[i] = A.addr[first[i]]
+            table_at = A.shared_at
+        if dpar is not None:
+            A.other[0] = int(np.array([dpar], np.float64).view(np.int64)[0])
+        else:
+            A.other[0] = swap if m_size is None else m_size
+        e = (A.run or A.bind())(_op_info(op)[2], table_at, n, A.other_at)
+        if e.error:
+            L.check(e)
+        o = 0
+        for i, p in enumerate(pdls):
+            if first[i] == i:
+                if p.state & L.NOMYDIMS:
+                    p.dtype, p.state, nd = _HEAD.unpack_from(mem, o)
+                    p.dims = list(_LONGS[nd].unpack_from(mem, o + _DIMS_AT))
+                    p.incs = list(_LONGS[nd].unpack_from(mem, o + _INCS_AT))
+                    p.offs = 0
+                    data = _DATA.unpack_from(mem, o + _DATA_AT)[0]
+                    p._buf = _Buf(data, p.nelem * _ITEMSIZE[p.dtype]) if data else None
+                else:
+                    p.state = _STATE.unpack_from(mem, o + _STATE_AT)[0]
+                if p.state & L.BADVAL:
+                    p._mark_parents_bad()
+            o += A.size
+        return pdls
     finally:
-        _spare.args = A
-
-
-def _call_in(A, op, pdls, swap, m_size, dpar):
-    """_call in the argument block A, which nothing else uses meanwhile"""
-    n = len(pdls)
-    if n > A.MAX:
-        raise PDLError(L.EUSERERROR, "pdlhip: %s: %d ndarrays" % (op, n))
-    mem, table_at, o = A.mem, A.table_at, 0
-    for p in pdls:
-        dims, incs, buf = p.dims, p.incs, p._buf
-        nd = len(dims)
-        if nd > L.MAXDIMS:
-            raise PDLError(L.EUSERERROR, "too many dims")
-        if len(incs) != nd:
-            incs = incs[:nd]
-        _STRUCTS[nd].pack_into(mem, o, p.dtype, p.state, nd, 0, *dims, *incs, p.offs,
-                               buf.ptr or 0 if buf is not None else 0)
-        if p.bids or p.badvalue_ is not None:
-            p._rest_to_c(A.pdls[o // A.size])
-        o += A.size
-    first = range(n)       # which struct each ndarray is: one passed twice is one pdl
-    if n > 1 and (pdls[0] is pdls[1] or n > 2 and len(set(map(id, pdls))) < n):
-        first = [next(j for j in range(n) if pdls[j] is p) for p in pdls]
-        for i in range(n):
-            A.shared[i] = A.addr[first[i]]
-        table_at = A.shared_at
-    if dpar is not None:
-        A.other[0] = int(np.array([dpar], np.float64).view(np.int64)[0])
-    else:
-        A.other[0] = swap if m_size is None else m_size
-    e = (A.run or A.bind())(_op_info(op)[2], table_at, n, A.other_at)
-    if e.error:
-        L.check(e)
-    o = 0
-    for i, p in enumerate(pdls):
-        if first[i] == i:
-            if p.state & L.NOMYDIMS:
-                p.dtype, p.state, nd = _HEAD.unpack_from(mem, o)
-                p.dims = list(_LONGS[nd].unpack_from(mem, o + _DIMS_AT))
-                p.incs = list(_LONGS[nd].unpack_from(mem, o + _INCS_AT))
-                p.offs = 0
-                data = _DATA.unpack_from(mem, o + _DATA_AT)[0]
-                p._buf = _Buf(data, p.nelem * _ITEMSIZE[p.dtype]) if data else None
-            else:
-                p.state = _STATE.unpack_from(mem, o + _STATE_AT)[0]
-            if p.state & L.BADVAL:
-                p._mark_parents_bad()
-        o += A.size
-    return pdls
+        if len(_spare) < 8:
+            _spare.append(A)
 
 
 def run(op, *pdls, swap=0, m_size=None, dpar=None):
