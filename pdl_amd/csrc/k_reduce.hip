@@ -448,8 +448,7 @@ __global__ __launch_bounds__(RT) void scan_seq(const Tin *__restrict__ a, RedPla
   auto out = [&](int64_t k) { return (Tout *)(sq_lds + 16 * G) + (int)(k & 1) * G * po; };
   auto in = [&](int64_t k) { return (Tin *)(sq_lds + 16 * G + 2 * G * po * sizeof(Tout)) + (int)(k & 1) * G * pi; };
   const int tid = threadIdx.x, lc = __builtin_ctz(C), lg = __builtin_ctz(G);
-  const int64_t e0 = grid_block() * G;
-  if (e0 >= p.nout) return;
+  const int64_t e0 = (int64_t)blockIdx.x * G;
   const int rows = p.nout - e0 < G ? (int)(p.nout - e0) : G;
   if (tid < rows) {
     int64_t off[MAXP];
@@ -615,8 +614,19 @@ static hipError_t seq_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
   const size_t lds = 16 * (size_t)G + 2 * (size_t)G * (sizeof(Tin) * sq_pitch<Tin, Tout>(C, one) +
                                                        sizeof(Tout) * sq_pitch<Tout, Tout>(C, one));
   const int64_t blocks = (p.nout + G - 1) / G;
-  if (blocks >= ((int64_t)1 << 31)) return hipErrorInvalidConfiguration;
-  const dim3 grid = grid_of(blocks);
+  if (blocks >= GRID_BLOCKS) {   // two halves of the longest broadcast dim
+    int d = 0;
+    for (int k = 1; k < p.nd; k++) d = p.dims[k] > p.dims[d] ? k : d;
+    RedPlan lo = p, hi = p;
+    lo.dims[d] = p.dims[d] / 2;
+    hi.dims[d] = p.dims[d] - lo.dims[d];
+    lo.nout = p.nout / p.dims[d] * lo.dims[d];
+    hi.nout = p.nout - lo.nout;
+    for (int q = 0; q < p.npdl; q++) hi.off[q] += lo.dims[d] * p.inc[q][d];
+    const hipError_t e = seq_launch<OP, Tin, Tout, BAD>(lo, a, o, ba, s);
+    return e == hipSuccess ? seq_launch<OP, Tin, Tout, BAD>(hi, a, o, ba, s) : e;
+  }
+  const dim3 grid((unsigned)blocks);
   if (one)
     hipLaunchKernelGGL((scan_seq<OP, Tin, Tout, BAD, true>), grid, dim3(RT), lds, s, a, p, o, ba, G, C,
                        nfast(0) ? 1 : 0, nfast(1) ? 1 : 0);

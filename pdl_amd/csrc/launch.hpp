@@ -9,16 +9,11 @@
 namespace pdlhip {
 
 // A launch dimension holds fewer than 2^32 threads: more wrap without an
-// error and the blocks past them never run.  In one dimension that is fewer
-// than GRID_BLOCKS blocks of 256 threads; from there on grid_of lays them out
-// in rows of 2^20, the last of which runs past the last block.
+// error and the blocks past them never run.  That is fewer than GRID_BLOCKS
+// blocks of 256 threads; larger work is split on the host (a second grid
+// dimension makes a kernel's indices 64 bits wide and costs small work up to
+// 9%).
 constexpr int64_t GRID_BLOCKS = (int64_t)1 << 24;
-constexpr int GRID_ROW = 20;
-inline dim3 grid_of(int64_t blocks) {
-  if (blocks < GRID_BLOCKS) return dim3((unsigned)blocks);
-  return dim3(1u << GRID_ROW, (unsigned)((blocks + (1 << GRID_ROW) - 1) >> GRID_ROW));
-}
-__device__ __forceinline__ int64_t grid_block() { return ((int64_t)blockIdx.y << GRID_ROW) + blockIdx.x; }
 
 #define PDLHIP_FOR_EACH_TYPE(X) X(0) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10)
 
