@@ -278,7 +278,8 @@ __global__ __launch_bounds__(RT) void red_grid(const Tin *__restrict__ a, RedPla
 // (Ufunc.pd:127-132).  Few long rows are cut into chunks of a multiple of 4096
 // elements, a block each: scan_totals leaves every chunk's total, and a
 // chunk's scan starts from the totals before it (16 rows of 1000000 ints:
-// 520 us with a block per row, 13 + 24 with chunks).
+// 520 us with a block per row, 13 + 24 with chunks).  Whole rows (not CUT) are
+// a form of their own (4096 of 1000 ints: 15 us, 16 with the chunk's tests).
 constexpr int SC_IT = 16, SC_CH = RT * SC_IT;
 __device__ inline int sc_pad(int i) { return i + (i >> 4); }
 
@@ -299,7 +300,7 @@ __global__ __launch_bounds__(RT) void scan_totals(const Tin *__restrict__ a, Red
   if (threadIdx.x == 0) totals[blockIdx.x] = pt.s;
 }
 
-template <int OP, class Tin, class Tout, bool BAD>
+template <int OP, class Tin, class Tout, bool BAD, bool CUT>
 __global__ __launch_bounds__(RT) void scan_rows(const Tin *__restrict__ a, RedPlan p, Outs o, BadInfo ba, int64_t nchunk,
                                                 int64_t clen, const Tout *totals) {
   constexpr bool PR = (OP == R_CUMUPROD);
@@ -310,14 +311,14 @@ __global__ __launch_bounds__(RT) void scan_rows(const Tin *__restrict__ a, RedPl
   const Tin abv = bv_as<Tin>(ba.bv);
   const Tout obv = bv_as<Tout>(o.bv[0]);
   const Tout ident = PR ? Tout(1) : Tout(0);
-  for (int64_t q = blockIdx.x; q < p.nout * nchunk; q += gridDim.x) {
-    const int64_t e = nchunk == 1 ? q : q / nchunk, k = q - e * nchunk;
+  for (int64_t q = blockIdx.x; q < (CUT ? p.nout * nchunk : p.nout); q += gridDim.x) {
+    const int64_t e = CUT ? q / nchunk : q, k = CUT ? q - e * nchunk : 0;
     int64_t off[MAXP];
     out_offsets(p, e, off);
     const Tin *ap = a + off[0];
     Tout *bp = (Tout *)o.p[0] + off[1];
     Tout carry = ident;
-    if (k > 0) {   // the totals of the row's chunks before this one
+    if (CUT && k > 0) {   // the totals of the row's chunks before this one
       Tout t = ident;
       for (int64_t i = tid; i < k; i += RT) t = PR ? wmul(t, totals[e * nchunk + i]) : wadd(t, totals[e * nchunk + i]);
 #pragma unroll
@@ -331,8 +332,8 @@ __global__ __launch_bounds__(RT) void scan_rows(const Tin *__restrict__ a, RedPl
       for (int i = 0; i < RT / 64; i++) carry = PR ? wmul(carry, wsum[i]) : wadd(carry, wsum[i]);
       __syncthreads();
     }
-    const int64_t end = (k + 1) * clen < p.n ? (k + 1) * clen : p.n;
-    for (int64_t c0 = k * clen; c0 < end; c0 += SC_CH) {
+    const int64_t end = CUT && (k + 1) * clen < p.n ? (k + 1) * clen : p.n;
+    for (int64_t c0 = CUT ? k * clen : 0; c0 < end; c0 += SC_CH) {
       const int len = (end - c0 < SC_CH) ? (int)(end - c0) : SC_CH;
       // every load of the chunk is issued before the first LDS write
       Tin xv[SC_IT];
@@ -810,10 +811,12 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
     if constexpr ((OP == R_CUMUSUM || OP == R_CUMUPROD) && !IsFloat<Tout>::v) {
       if (p.inc_n[0] == 1 && p.inc_n[1] == 1 && p.n >= 256) {
         // rows of several chunks are cut while they alone leave CUs idle:
-        // about 2048 blocks in all, each of at least 8192 elements
+        // about 2048 blocks in all, each of at least 8192 elements.  From a
+        // row per CU on, reading everything twice costs more (500 rows of
+        // 40000 ints: 32 us, cut 43)
         int64_t nchunk = 1, clen = p.n;
         Tout *totals = nullptr;
-        if (p.nout < 512 && p.n >= 32768) {
+        if (p.nout < 256 && p.n >= 32768) {
           int64_t want = (2048 + p.nout - 1) / p.nout;
           clen = (p.n + want - 1) / want;
           clen = clen < 8192 ? 8192 : (clen + SC_CH - 1) / SC_CH * SC_CH;
@@ -825,8 +828,12 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
           hipLaunchKernelGGL((scan_totals<OP, Tin, Tout, BAD>), dim3((unsigned)(p.nout * nchunk)), dim3(RT), 0, s, a, p,
                              ba, nchunk, clen, totals);
         const int64_t blocks = p.nout * nchunk < 65536 ? p.nout * nchunk : 65536;
-        hipLaunchKernelGGL((scan_rows<OP, Tin, Tout, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba, nchunk,
-                           clen, totals);
+        if (totals)
+          hipLaunchKernelGGL((scan_rows<OP, Tin, Tout, BAD, true>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
+                             nchunk, clen, totals);
+        else
+          hipLaunchKernelGGL((scan_rows<OP, Tin, Tout, BAD, false>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
+                             nchunk, clen, totals);
         const hipError_t err = hipGetLastError();
         if (totals) partials_free(totals);
         return err;
