@@ -609,6 +609,9 @@ static hipError_t seq_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
   while (C > 32 && C / 2 >= p.n) C /= 2;
   // more rows where they are short
   while (G < 64 && G * C * 2 <= E && (int64_t)G * 2 * 256 <= p.nout) G *= 2;
+  // (the shortest rows: no more than a group of 16; 100000 of 16 ints 13.3 us,
+  // 14.4 with 32)
+  if (G > 1 && p.n <= 16) C = 16;
   const bool one = G == 1;
   auto mag = [](int64_t x) { return x < 0 ? -x : x; };
   auto nfast = [&](int q) { return p.nout == 1 || p.nd == 0 || mag(p.inc_n[q]) <= mag(p.inc[q][0]); };
