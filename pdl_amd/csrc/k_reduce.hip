@@ -18,8 +18,8 @@
 //   scan   integer scans of unit-stride rows: blocks scan chunks through LDS.
 //   seq    scans in PDL's order: a lane per row in LDS, other waves moving.
 //   thread one thread per output walking n in index order (float products,
-//          *_n_ind): adjacent threads read adjacent addresses when the
-//          broadcast dim 0 is the contiguous one.
+//          *_n_ind, the shortest rows and columns): adjacent threads read
+//          adjacent addresses when the broadcast dim 0 is the contiguous one.
 //
 // Semantics kept exactly: integer sums/products wrap in the output type
 // (any order gives PDL's bits), min/max follow PDL's rules (a NaN never
@@ -260,12 +260,12 @@ __global__ __launch_bounds__(RT) void red_grid(const Tin *__restrict__ a, RedPla
         part_push<OP, Tin, Tacc>(pt, x[u], q);
       }
     }
-    block_tree<OP>(pt, sh, in, r, R, NFAST ? 1 : LE);
+    if (R > 1) block_tree<OP>(pt, sh, in, r, R, NFAST ? 1 : LE);
     if (in && r == 0) {
       if (nchunk == 1) part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
       else parts[e * nchunk + k] = pt;
     }
-    __syncthreads();   // sh is refilled for the next group
+    if (R > 1) __syncthreads();   // sh is refilled for the next group
   }
 }
 
@@ -689,8 +689,26 @@ __global__ __launch_bounds__(RT) void red_thread(const Tin *__restrict__ a, RedP
       Tout v = (Tout)tmp;
       if (BAD && !any) v = bv_as<Tout>(o.bv[0]);
       put<Tout>(o.p[0], off[1], v);
+    } else {
+      Part<Tin, Tacc> pt;
+      part_init<OP, Tin, Tacc>(pt);
+      for (int64_t i = 0; i < n; i++) {
+        const Tin x = ap[i * ia];
+        if constexpr (BAD) { if (isbad(x, abv, ba.isnan)) continue; }
+        part_push<OP, Tin, Tacc>(pt, x, i);
+      }
+      part_store<OP, Tin, Tout, Tacc>(pt, o, off, BAD);
     }
   }
+}
+
+template <int OP, class Tin, class Tout, class Tacc, bool BAD>
+static hipError_t thread_launch(const RedPlan &p, const Tin *a, const Outs &o, const BadInfo &ba, int *flag,
+                                hipStream_t s) {
+  int64_t blocks = (p.nout + RT - 1) / RT;
+  if (blocks > 65536) blocks = 65536;
+  hipLaunchKernelGGL((red_thread<OP, Tin, Tout, Tacc, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba, flag);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- dispatch
@@ -704,11 +722,21 @@ static hipError_t grid_launch(const RedPlan &p, const Tin *a, const Outs &o, con
   const int64_t in0 = p.inc_n[0] < 0 ? -p.inc_n[0] : p.inc_n[0];
   const int64_t ie0 = p.nd == 0 || p.nout == 1 ? INT64_MAX : (p.inc[0][0] < 0 ? -p.inc[0][0] : p.inc[0][0]);
   const bool nfast = in0 < ie0;
+  // The shortest rows, and short columns of outputs that fill the chip: the
+  // plain loop of red_thread, whose block holds nothing but its outputs
+  // (1000000 rows of 5 floats 8 us, here 12; 3000000 columns of 10 floats 29,
+  // here 35; rows of 8 doubles 24 and 17, columns of 33 doubles 20 and 17).
+  if (nfast ? p.n < 8 || p.n * (int64_t)sizeof(Tin) <= 16 : p.n < 16 && p.nout >= 262144)
+    return thread_launch<OP, Tin, Tout, Tacc, BAD>(p, a, o, ba, nullptr, s);
   int LE, R;
   if (nfast) {
-    // at least four elements per thread before a second thread helps
+    // a thread for rows up to 64 bytes, then one for every 16 elements: with
+    // fewer to load, the tree costs a thread more than it saves (1000000 rows
+    // of 63 floats: 63 us, with a thread per four elements 187; of 16 floats
+    // 33 and 44)
     R = 1;
-    while (R < 64 && R * 4 < p.n) R *= 2;
+    if (p.n * (int64_t)sizeof(Tin) > 64)
+      while (R < 64 && R * 16 <= p.n) R *= 2;
     LE = RT / R;
     if (p.nout < LE) {   // fewer outputs than that: more threads along n
       LE = (int)p.nout;
@@ -845,11 +873,7 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
     if (p.n == 0) return hipSuccess;
     return seq_launch<OP, Tin, Tout, BAD>(p, a, o, ba, s);
   } else {
-    int64_t blocks = (p.nout + RT - 1) / RT;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL((red_thread<OP, Tin, Tout, Tacc, BAD>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o, ba,
-                       flag);
-    return hipGetLastError();
+    return thread_launch<OP, Tin, Tout, Tacc, BAD>(p, a, o, ba, flag, s);
   }
 }
 
