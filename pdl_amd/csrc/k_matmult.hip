@@ -22,6 +22,8 @@ namespace pdlhip {
 
 hipError_t launch_mfma_f32(const MmPlan &p, const float *a, const float *b, float *c, int mode, hipStream_t s);
 hipError_t launch_tile_f64(const MmPlan &p, const double *a, const double *b, double *c, hipStream_t s);
+bool wide_f64(const MmPlan &p);
+hipError_t launch_wide_f64(const MmPlan &p, const double *a, const double *b, double *c, hipStream_t s);
 hipError_t launch_tile_f32(const MmPlan &p, const float *a, const float *b, float *c, hipStream_t s);
 bool tile_takes_f32(const MmPlan &p);   // whether the default mode runs p on launch_tile_f32
 
@@ -188,7 +190,8 @@ static hipError_t matmult_T(const MmPlan &p, const void *va, const void *vb, voi
   if constexpr (sizeof(T) == 8 && IsFloat<T>::v) {
     // the default mode runs double products on the FP64 matrix cores
     if (mode == PDLHIP_MM_SPLIT16 || mode == PDLHIP_MM_FP8) {
-      hipError_t e = launch_tile_f64(p, (const double *)a, (const double *)b, (double *)c, s);
+      hipError_t e = wide_f64(p) ? launch_wide_f64(p, (const double *)a, (const double *)b, (double *)c, s)
+                                 : launch_tile_f64(p, (const double *)a, (const double *)b, (double *)c, s);
       if (e != hipErrorNotSupported) return e;
     }
   }
