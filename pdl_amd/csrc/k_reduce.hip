@@ -813,11 +813,21 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
         if (!p.scratch) scratch_free(parts);
         return err;
       }
-      // a wave per row where the rows fill the chip (sixteen waves per CU) or
-      // are short; else enough waves per row, each with about four 16-byte
-      // loads per lane
-      const int64_t loads = (int64_t)(row_bytes / 16 / 64);
-      if (p.nout >= 4096 || loads < 8) {
+      // Waves per row: with more than about 5000 in all they run in turns and
+      // only add their joining, so sixteen a row up to 256 rows, four up to
+      // 1280, one beyond; more where a lane would have very many elements,
+      // fewer where not even that many loads.  Both sides, us with 1 / 4 / 16:
+      // maximum of 256 rows of 25600 shorts 23 / 10.6 / 7.7, 600 of 12800 floats
+      // 15 / 9 / 20, 1500 of 8192 shorts 12.9 / 9.6, of 4096 floats 8.6 / 9.6,
+      // 2676 of 2048 floats 7 / 13.5, 3500 of 1024 doubles 7 / 15.6, 2048 of
+      // 51200 shorts 53 / 42 / 60.
+      const int64_t loads = (int64_t)(row_bytes / 16 / 64), each = p.n / 64;   // per lane of one wave
+      const int waves = (p.nout <= 256 && loads >= 32) || (p.nout <= 640 && each >= 1600) ? 16
+                        : (p.nout <= 1280 && loads >= 8) || (p.nout <= 1600 && each >= 100) ||
+                              (p.nout < 4096 && each >= 300)
+                            ? 4
+                            : 1;
+      if (waves == 1) {
         int64_t blocks = (p.nout + 3) / 4;
         if (blocks > 65536) blocks = 65536;
         bool on16 = (uintptr_t)(a + p.off[0]) % 16 == 0;
@@ -828,7 +838,7 @@ static hipError_t red_launch(const RedPlan &p, const Tin *a, const Outs &o, cons
         else
           hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 1>), dim3((unsigned)blocks), dim3(RT), 0, s, a, p, o,
                              ba, stream);
-      } else if (p.nout >= 1024 || loads < 32) {
+      } else if (waves == 4) {
         hipLaunchKernelGGL((red_wave<OP, Tin, Tout, Tacc, BAD, 4>), dim3((unsigned)p.nout), dim3(RT), 0, s, a, p, o, ba,
                            stream);
       } else {

@@ -32,6 +32,19 @@ def test_short_rows(t, n):
         both_ways(t, rand(t, (rows, n), rng), [])
 
 
+@pytest.mark.parametrize("rows,n", [(256, 8200), (257, 8200), (1280, 2048), (1281, 2048), (1600, 6400), (1601, 6400), (300, 102401), (640, 102400),
+                                    (641, 102400), (4095, 19200), (4096, 19200), (4095, 19199), (40, 2047)],
+                         ids=lambda s: str(s))
+@pytest.mark.parametrize("t", [O.B, O.F], ids=lambda t: O.TYPE_NAMES[t])
+def test_waves_per_row(t, rows, n):
+    if rows * n > 2 ** 25 and t != O.B:
+        pytest.skip("the same path as the bytes; the oracle's pass over it is long")
+    rng = np.random.default_rng(rows)
+    A = pair(rand(t, (rows, n), rng), t)
+    for op in ("sumover", "maximum_ind"):
+        check(op, t, A)
+
+
 @pytest.mark.parametrize("n", [1, 4, 15, 16, 17])
 @pytest.mark.parametrize("cols", [262143, 262144, 262147])
 @pytest.mark.parametrize("t", [O.S, O.D], ids=lambda t: O.TYPE_NAMES[t])
