@@ -358,10 +358,10 @@ pdlhip_error pdlhip_graph_destroy(void *graph);
  *   SPLIT16   default; double: FP64 MFMA from 8 per side; float: by its
  *             sizes alone, either FP32 MFMA with sums in parts of a few k
  *             (from 8 per side), or an FP16 hi/lo split, 3 MFMA products,
- *             FP32 accumulate: beyond 3e10 operations, below that where it is
- *             the faster one (from about 7e9), and for products with 33..64
- *             per side, but not with another side below 64 or fewer than 32
- *             k; sides below 8 as FP32
+ *             FP32 accumulate (products with 33..64 per side; and single
+ *             ones with sides from 64 and 32 k up, where that is estimated
+ *             to be faster, from about 7e9 operations, or beyond 3e10);
+ *             sides below 8 as FP32
  *   FP32      plain SIMT kernel with fused multiply-add (float and double)
  *   PDLORDER  SIMT, multiply then add in ascending t: bit-identical to the
  *             reference's loop

@@ -30,8 +30,9 @@
 // v_mfma_f32_16x16x32_fp8_fp8.  Only non-finite rows are recomputed: the
 // FP8 path is approximate by design.
 //
-// Layout: packed operands are [row][Kp] with K contiguous, rows padded to the
-// block tile and K to the k step (zeros).
+// Layout: rows are padded to the block tile and K to the k step (zeros); FP16
+// operands are packed as pieces of 32 rows x 16 k, hi and lo (mfma_common.hpp,
+// panel_at), FP8 ones as [row][Kp] with K contiguous.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -206,8 +207,8 @@ __device__ __forceinline__ float pack8(const float (&x)[8], float sc, half_t *hl
   return ex;
 }
 
-// pack a (R x K) operand into hi/lo fp16 [Rp][Kp] through a 64x64 LDS tile so
-// that both the strided read and the K-contiguous write are coalesced
+// pack a (R x K) operand into the FP16 panels (or FP8 rows) through a 64x64 LDS
+// tile so that both the strided read and the write along K are coalesced
 template <bool FP8>
 __global__ __launch_bounds__(256) void pack_tile(const float *__restrict__ src, int64_t o, int64_t inc_r,
                                                  int64_t inc_k, int64_t R, int64_t K, int64_t Kp,

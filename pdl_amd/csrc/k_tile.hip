@@ -6,9 +6,9 @@
 // are small: 64x64 of C per block of 4 waves keeps four blocks resident per
 // CU, whose waves cover each other's loads and barriers, and cuts a product
 // into enough blocks for 256 CUs.  Double: 4096^3 2.09 ms, 65.8 TFLOP/s
-// (128x128 blocks of the same kernel 2.33 ms, 128x64 2.28); 1500^3 148 us (123
-// where the operands change from call to call; before, 144 blocks of 128x128:
-// 280); 512^3 18 us (the SIMT kernel: 85).  One stage of loads in flight
+// (128x128 blocks of the same kernel 2.33 ms, 128x64 2.28); 1500^3 132 + 4 us
+// for the join in a trace, 119 a call among others (before, 144 blocks of
+// 128x128: 277); 512^3 18 us (the SIMT kernel: 85).  One stage of loads in flight
 // instead of two: 59 instead of 54 us at 1024^3, where a CU has one block.
 // Float: 1024^3 30 us (packed for the FP16 split 70), 300^3 12 (46), 1413 x
 // 1452 x 19 16 (the SIMT kernel 184), 128 x 8192 x 128 23 (174), 65536 of 32^3
