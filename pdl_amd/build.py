@@ -36,7 +36,10 @@ VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
 def known(flags):
     """whether hipcc takes the flags (an empty source compiles with them)"""
     cmd = [HIPCC, "--offload-arch=" + ARCH] + flags + ["--cuda-device-only", "-x", "hip", "-S", os.devnull, "-o", os.devnull]
-    return subprocess.run(cmd, capture_output=True).returncode == 0
+    try:
+        return subprocess.run(cmd, capture_output=True).returncode == 0
+    except OSError:
+        return False  # no hipcc: the units can still be listed
 
 
 def units():
