@@ -32,13 +32,14 @@ def test_short_rows(t, n):
         both_ways(t, rand(t, (rows, n), rng), [])
 
 
-@pytest.mark.parametrize("rows,n", [(256, 8200), (257, 8200), (1280, 2048), (1281, 2048), (1600, 6400), (1601, 6400), (300, 102401), (640, 102400),
-                                    (641, 102400), (4095, 19200), (4096, 19200), (4095, 19199), (40, 2047)],
+WAVES = [(256, 8200), (257, 8200), (1280, 2048), (1281, 2048), (1600, 6400), (1601, 6400), (300, 102401), (640, 102400), (641, 102400),
+         (4095, 19200), (4096, 19200), (4095, 19199), (40, 2047)]
+
+
+# the longest as bytes only: the same path, and the oracle's pass over them is long
+@pytest.mark.parametrize("t,rows,n", [(t, r, n) for t in (O.B, O.F) for r, n in WAVES if t == O.B or r * n <= 2 ** 25],
                          ids=lambda s: str(s))
-@pytest.mark.parametrize("t", [O.B, O.F], ids=lambda t: O.TYPE_NAMES[t])
 def test_waves_per_row(t, rows, n):
-    if rows * n > 2 ** 25 and t != O.B:
-        pytest.skip("the same path as the bytes; the oracle's pass over it is long")
     rng = np.random.default_rng(rows)
     A = pair(rand(t, (rows, n), rng), t)
     for op in ("sumover", "maximum_ind"):
